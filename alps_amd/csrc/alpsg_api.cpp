@@ -77,14 +77,16 @@ hipError_t launch_round(hipStream_t st, int nchr, int RB, int RC, const ProbDev 
 hipError_t launch_assemble_osc(hipStream_t st, const ProbDev *prob, int nspec, int nom, int W, int RB,
                                double2 *om, const double2 *chiA, const double2 *chiB, double2 *det,
                                alpsg_osc::OscMachine *S, int *round_ctr, int *remaining);
-hipError_t launch_rel(hipStream_t st, const ProbDev *prob, int nspec, int nmaxR, int NB, int nom,
-                      const double2 *om, const int *active, double2 *chiR, double2 *lowR,
-                      int *flags, int *err, const int *pidx = nullptr);
-int rel_slots(int NB, int nmaxR);
+hipError_t launch_rel(hipStream_t st, const ProbDev *prob, int nspec, int nmaxR, RelSplit sp,
+                      int nom, const double2 *om, const int *active, double2 *chiR, double2 *lowR,
+                      int *flags, int *err);
+RelSplit rel_split(int nom);
+int rel_slots(RelSplit sp, int nmaxR);
+int rel_low_slots(RelSplit sp);
 hipError_t launch_assemble(hipStream_t st, const ProbDev *prob, int nspec, int nom, int W, int RB,
                            const double2 *om, const int *active, const double2 *chiA,
                            const double2 *chiB, const double2 *lowA, const double2 *lowB,
-                           const double2 *chiR, int RR, const double2 *lowR, double2 *det,
+                           const double2 *chiR, int RR, const double2 *lowR, int LR, double2 *det,
                            double2 *chi, double2 *low, double2 *wave, const int *pidx = nullptr);
 
 namespace {
@@ -262,7 +264,6 @@ struct alpsg_ctx {
   DevBuf<double> gtab;
   DevBuf<double2> chiR_d, lowR_d;
   DevBuf<int> flags_d, err_d;
-  int rel_NB = 1;
   std::vector<double> current_int;  // parallel current density per species
   bool have_current = false;
   // launch shapes chosen by alpsg_autotune (or pinned by alpsg_set_shape),
@@ -427,22 +428,23 @@ int disp_chain(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_dev
   if (h->any_bm)
     HIPCHK(launch_nhds(h->st, h->prob_d.p, ns, n, om_dev, active_dev, B.chiA,
                        want_low ? B.lowA : nullptr));
-  int RR = 0;
+  int RR = 0, LR = 0;
   if (h->any_rel) {
     const int nmaxR = h->prob.nmaxR;
-    const int NB = std::max(1, std::min(2 * nmaxR + 1, 1024 / std::max(n, 1)));
-    RR = rel_slots(NB, nmaxR);
+    const RelSplit sp = rel_split(n);
+    RR = rel_slots(sp, nmaxR);
+    LR = rel_low_slots(sp);
     HIPCHK(h->chiR_d.ensure((size_t)RR * ns * 6 * n));
     HIPCHK(h->flags_d.ensure((size_t)n * ns * (2 * nmaxR + 1)));
-    if (want_low) HIPCHK(h->lowR_d.ensure((size_t)n * ns * 18));
-    HIPCHK(launch_rel(h->st, h->prob_d.p, ns, nmaxR, NB, n, om_dev, active_dev, h->chiR_d.p,
+    if (want_low) HIPCHK(h->lowR_d.ensure((size_t)LR * n * ns * 18));
+    HIPCHK(launch_rel(h->st, h->prob_d.p, ns, nmaxR, sp, n, om_dev, active_dev, h->chiR_d.p,
                       want_low ? h->lowR_d.p : nullptr, h->flags_d.p, h->err_d.p));
   }
   HIPCHK(hipEventRecord(h->ev_res, h->st));
   HIPCHK(launch_assemble(h->st, h->prob_d.p, ns, n, TWa, sh.rb, om_dev, active_dev, B.chiA, B.chiB,
                          want_low ? B.lowA : nullptr, want_low ? B.lowB : nullptr,
                          RR ? h->chiR_d.p : nullptr, RR, (RR && want_low) ? h->lowR_d.p : nullptr,
-                         B.det, want_chi ? B.chi : nullptr, want_low ? B.low : nullptr,
+                         LR, B.det, want_chi ? B.chi : nullptr, want_low ? B.low : nullptr,
                          want_wave ? B.wave : nullptr));
   return ALPSG_OK;
 }
@@ -709,7 +711,7 @@ int graph_disp(alpsg_ctx *h, int n, const double *om, double *det) {
                               h->lgen);
     if (e == hipSuccess)
       e = launch_assemble(h->st, h->prob_d.p, ns, n, REQ_TW / REQ_W, sh.rb, h->om_d.p, nullptr, h->chiA_d.p,
-                          h->chiB_d.p, nullptr, nullptr, nullptr, 0, nullptr, h->det_d.p, nullptr,
+                          h->chiB_d.p, nullptr, nullptr, nullptr, 0, nullptr, 0, h->det_d.p, nullptr,
                           nullptr, nullptr);
     if (e == hipSuccess)
       e = hipMemcpyAsync(h->det_pin.p, h->det_d.p, sizeof(double2) * n, hipMemcpyDeviceToHost,
@@ -915,7 +917,7 @@ int osc_graph_batch(alpsg_ctx *h, const alpsg_root_params *rp, int n, cplx *om, 
                             h->chiB_d.p, nullptr, h->lgen, nullptr, h->P);
       if (e == hipSuccess)
         e = launch_assemble(h->st, h->prob_d.p, ns, n, TW, sh.rb, h->om_d.p, nullptr, h->chiA_d.p,
-                            h->chiB_d.p, nullptr, nullptr, nullptr, 0, nullptr, h->det_d.p, nullptr,
+                            h->chiB_d.p, nullptr, nullptr, nullptr, 0, nullptr, 0, h->det_d.p, nullptr,
                             nullptr, nullptr);
       if (e == hipSuccess)
         e = launch_osc_round(h->st, n, h->osc_d.p, h->det_d.p, h->om_d.p, h->oscctl_d.p,

@@ -105,6 +105,12 @@ struct ProbDev {
   SpecDev sp[ALPSG_DMAXSPEC];
 };
 
+// How a batch splits a relativistic species' harmonics (rel_split): workgroups
+// per harmonic group of k_rel_nonres and per harmonic of k_rel_res.
+struct RelSplit {
+  int B, RS;
+};
+
 // ---------------------------------------------------------------------------
 // Small complex helpers (double2 = (re, im)).
 // ---------------------------------------------------------------------------

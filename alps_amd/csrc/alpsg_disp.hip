@@ -1661,14 +1661,15 @@ __global__ __launch_bounds__(64) void k_resonant_all(const ProbDev *__restrict__
 // ---------------------------------------------------------------------------
 // k_assemble: a workgroup of 256 threads handles 256/(6 nspec) omegas; thread
 // (omega, s, k) sums the partials of chi_sk, then one thread per omega forms
-// the dielectric tensor, the wave tensor and det D.
+// the dielectric tensor, the wave tensor and det D.  LR: the slots of lowR, or
+// -1 where chiR holds the served form's slots (rel_ord_slots).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void assemble_block(
     int blk, const ProbDev *__restrict__ probp, int nom, int W, int RB,
     const double2 *__restrict__ om_in, const int *__restrict__ active,
     const double2 *__restrict__ chiA, const double2 *__restrict__ chiB,
     const double2 *__restrict__ lowA, const double2 *__restrict__ lowB,
-    const double2 *__restrict__ chiR, int RR, const double2 *__restrict__ lowR,
+    const double2 *__restrict__ chiR, int RR, const double2 *__restrict__ lowR, int LR,
     double2 *__restrict__ det_out, double2 *__restrict__ chi_out, double2 *__restrict__ low_out,
     double2 *__restrict__ wave_out, int nspec, const int *__restrict__ pidx,
     double2 *det_lds = nullptr) {
@@ -1700,11 +1701,38 @@ __device__ __forceinline__ void assemble_block(
 #pragma unroll
       for (int u = 0; u < 16; ++u) v = v + mk(buf[u].x, buf[u].y);
     }
-    if (Pd.sp[s].rel)  // relativistic species: the partial slots of k_rel_nonres / k_rel_res
-      for (int j = 0; j < RR; ++j) {
-        const double2 a = chiR[((size_t)(j * nspec + s) * 6 + k) * nom + iom];
-        v = v + mk(a.x, a.y);
+    if (Pd.sp[s].rel) {
+      // relativistic species: the partial slots of the k_rel kernels, in
+      // batches of 16 loads
+      auto slot = [&](int j) { return chiR[((size_t)(j * nspec + s) * 6 + k) * nom + iom]; };
+      int j0 = 0;
+      if (LR < 0) {
+        // the served form: the non-resonant harmonics first, in four groups of
+        // every fourth harmonic from -nmax
+        const int nm = Pd.sp[s].nmax_rel, z0 = Pd.nmaxR - nm, z1 = Pd.nmaxR + nm;
+        for (int g = 0; g < 4; ++g) {
+          cd r = mk(0.0, 0.0);
+          for (int base = z0 + g; base <= z1; base += 64) {
+            double2 buf[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+              buf[u] = base + 4 * u <= z1 ? slot(base + 4 * u) : make_double2(0.0, 0.0);
+#pragma unroll
+            for (int u = 0; u < 16; ++u) r = r + mk(buf[u].x, buf[u].y);
+          }
+          v = v + r;
+        }
+        j0 = RR / 3;
       }
+      for (int base = j0; base < RR; base += 16) {
+        double2 buf[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          buf[u] = base + u < RR ? slot(base + u) : make_double2(0.0, 0.0);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v = v + mk(buf[u].x, buf[u].y);
+      }
+    }
     lchi[t] = make_double2(v.re, v.im);
   }
   __syncthreads();
@@ -1749,10 +1777,13 @@ __device__ __forceinline__ void assemble_block(
           if (qq == 1 && (q == 0 || q == 3 || q == 4)) continue;
           cd tt;
           if (S.rel) {
-            // relativistic: one of k_rel_nonres / k_rel_res wrote the term; the
+            // relativistic: the parts k_rel_nonres, k_rel_res and k_rel_landau wrote; the
             // ee term goes into chi only (ALPS_fns.f90:481-486)
-            const double2 a = lowR[((size_t)iom * nspec + sp) * 18 + 6 * qq + q];
-            tt = mk(a.x, a.y);
+            tt = mk(0.0, 0.0);
+            for (int j = 0; j < LR; ++j) {
+              const double2 a = lowR[(((size_t)j * nom + iom) * nspec + sp) * 18 + 6 * qq + q];
+              tt = tt + mk(a.x, a.y);
+            }
           } else {
             const double2 a = lowA[((size_t)iom * nspec + sp) * 18 + 6 * qq + q];
             tt = mk(a.x, a.y);
@@ -1812,11 +1843,11 @@ __global__ __launch_bounds__(256) void k_assemble(
     const int *__restrict__ active, const double2 *__restrict__ chiA,
     const double2 *__restrict__ chiB, const double2 *__restrict__ lowA,
     const double2 *__restrict__ lowB, const double2 *__restrict__ chiR, int RR,
-    const double2 *__restrict__ lowR, double2 *__restrict__ det_out, double2 *__restrict__ chi_out,
+    const double2 *__restrict__ lowR, int LR, double2 *__restrict__ det_out, double2 *__restrict__ chi_out,
     double2 *__restrict__ low_out, double2 *__restrict__ wave_out, int nspec,
     const int *__restrict__ pidx) {
   assemble_block(blockIdx.x, probp, nom, W, RB, om_in, active, chiA, chiB, lowA, lowB, chiR, RR,
-                 lowR, det_out, chi_out, low_out, wave_out, nspec, pidx);
+                 lowR, LR, det_out, chi_out, low_out, wave_out, nspec, pidx);
 }
 
 // ---------------------------------------------------------------------------
@@ -1906,13 +1937,13 @@ hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob,
 hipError_t launch_assemble(hipStream_t st, const ProbDev *prob, int nspec, int nom, int W, int RB,
                            const double2 *om, const int *active, const double2 *chiA,
                            const double2 *chiB, const double2 *lowA, const double2 *lowB,
-                           const double2 *chiR, int RR, const double2 *lowR, double2 *det,
+                           const double2 *chiR, int RR, const double2 *lowR, int LR, double2 *det,
                            double2 *chi, double2 *low, double2 *wave, const int *pidx) {
   if (nom <= 0) return hipSuccess;
   const int per = 6 * nspec;
   const int opb = 256 / per;
   hipLaunchKernelGGL(k_assemble, dim3((nom + opb - 1) / opb), dim3(256), 0, st, prob, nom, W, RB,
-                     om, active, chiA, chiB, lowA, lowB, chiR, RR, lowR, det, chi, low, wave, nspec,
+                     om, active, chiA, chiB, lowA, lowB, chiR, RR, lowR, LR, det, chi, low, wave, nspec,
                      pidx);
   return hipGetLastError();
 }
@@ -2083,7 +2114,7 @@ __global__ __launch_bounds__(256) void k_assemble_osc(
   const int opb = 256 / (6 * nspec);
   for (int blk = 0; blk * opb < nom; ++blk) {
     assemble_block(blk, probp, nom, W, RB, om_in, nullptr, chiA, chiB, nullptr, nullptr, nullptr, 0,
-                   nullptr, det, nullptr, nullptr, nullptr, nspec, nullptr, det_l);
+                   nullptr, 0, det, nullptr, nullptr, nullptr, nspec, nullptr, det_l);
     __syncthreads();
   }
   int more = 0;

@@ -79,17 +79,17 @@ hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob,
 hipError_t launch_assemble(hipStream_t st, const ProbDev *prob, int nspec, int nom, int W, int RB,
                            const double2 *om, const int *active, const double2 *chiA,
                            const double2 *chiB, const double2 *lowA, const double2 *lowB,
-                           const double2 *chiR, int RR, const double2 *lowR, double2 *det,
+                           const double2 *chiR, int RR, const double2 *lowR, int LR, double2 *det,
                            double2 *chi, double2 *low, double2 *wave, const int *pidx);
 hipError_t launch_nhds(hipStream_t st, const ProbDev *prob, int nspec, int nom, const double2 *om,
                        const int *active, double2 *chiA, double2 *lowA, const int *pidx);
 int nhds_tables(double z, int bm_nmax, double bessel_zero, std::vector<double2> &tab);
 hipError_t launch_rel_bessel(hipStream_t st, int npts, int nmax, double zfac, const double *grel,
                              const double *pbrel, const int *mtab, double *out);
-hipError_t launch_rel(hipStream_t st, const ProbDev *prob, int nspec, int nmaxR, int NB, int nom,
-                      const double2 *om, const int *active, double2 *chiR, double2 *lowR,
-                      int *flags, int *err, const int *pidx);
-int rel_slots(int NB, int nmaxR);
+hipError_t launch_rel_ord(hipStream_t st, const ProbDev *prob, int nspec, int nmaxR, int nom,
+                          const double2 *om, double2 *chiR, int *flags, int *err,
+                          const int *pidx);
+int rel_ord_slots(int nmaxR);
 
 namespace {
 
@@ -116,7 +116,6 @@ constexpr int SW_NCH = SW_SHAPE[0], SW_W = SW_SHAPE[1], SW_RC = SW_SHAPE[2], SW_
 #define ALPSG_SERVE_RB 8
 #endif
 constexpr int RS_RB = ALPSG_SERVE_RB;
-constexpr int REL_NB = 4;  // harmonic blocks of k_rel_nonres in a pass (fixed, as every shape here)
 constexpr size_t ALIGN = 256;
 constexpr int MAX_JOBS = 8192;               // (request, species) jobs per table launch
 constexpr size_t STAGE_CAP = (size_t)1 << 20;  // doubles read back per pass (int_ee, max|J_n|)
@@ -1057,7 +1056,7 @@ int server_pass(alpsg_server *S) {
       for (i1 = i0; i1 < nb && act[i1]->pl->nspec == ns; ++i1) relmax = std::max(relmax, act[i1]->nmaxR);
       if (relmax < 0) continue;
       const size_t n = (size_t)(i1 - i0);
-      need_r = std::max(need_r, n * rel_slots(REL_NB, relmax) * ns * 6);
+      need_r = std::max(need_r, n * rel_ord_slots(relmax) * ns * 6);
       need_f = std::max(need_f, n * ns * (size_t)(2 * relmax + 1));
       pass_rel = true;
     }
@@ -1106,19 +1105,19 @@ int server_pass(alpsg_server *S) {
       if (bm)
         SCHK(launch_nhds(S->st, S->probs_d, ns, n, S->om_d + i0, nullptr, S->chiA, nullptr,
                          S->pidx_d + i0));
-      // relativistic species: REL_NB + 2 relmax + 1 partial slots; an omega whose
+      // relativistic species: rel_ord_slots(relmax) partial slots; an omega whose
       // problem has fewer harmonics gets zeros in the slots past its own
       int RR = 0;
       if (ev) SCHK(hipEventRecord(ev[2], S->st));
       if (relmax >= 0) {
-        RR = rel_slots(REL_NB, relmax);
-        SCHK(launch_rel(S->st, S->probs_d, ns, relmax, REL_NB, n, S->om_d + i0, nullptr, S->chiR,
-                        nullptr, S->flags_d, S->err_d + i0, S->pidx_d + i0));
+        RR = rel_ord_slots(relmax);
+        SCHK(launch_rel_ord(S->st, S->probs_d, ns, relmax, n, S->om_d + i0, S->chiR, S->flags_d,
+                            S->err_d + i0, S->pidx_d + i0));
       }
       if (ev) SCHK(hipEventRecord(ev[3], S->st));
       SCHK(launch_assemble(S->st, S->probs_d, ns, n, SW_W * SW_RC, RS_RB, S->om_d + i0, nullptr,
                            S->chiA, S->chiB, nullptr, nullptr, RR ? S->chiR : nullptr, RR, nullptr,
-                           S->det_d + i0, nullptr, nullptr, nullptr, S->pidx_d + i0));
+                           -1, S->det_d + i0, nullptr, nullptr, nullptr, S->pidx_d + i0));
       if (ev) SCHK(hipEventRecord(ev[4], S->st));
       i0 = i1;
     }
