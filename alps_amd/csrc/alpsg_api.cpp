@@ -356,14 +356,45 @@ int size_bucket(int n) {
   return b;
 }
 
-LaunchShape pick_shape(int n) {
-  if (n >= 32768) return {1, 4, 1, 16, 1};
-  if (n >= 8192) return {2, 4, 1, 16, 1};
-  if (n >= 2048) return {8, 4, 1, 32, 1};
-  if (n >= 256) return {16, 8, 1, 32, 2};
-  if (n >= 32) return {32, 8, 2, 64, 4};
-  return {64, 8, 4, 64, 8};
+// The shape of a batch that has not been tuned; rows: the harmonic row pairs
+// of its species (no more wavefronts per omega block than row pairs).
+//
+// From 1024 omegas the sweep takes one lane per omega: its node records are
+// wave-uniform scalar loads, and only it sums far rows by their series and near
+// ones in the split form.  That leaves n / 64 blocks, so the row pairs are
+// dealt to as many wavefronts as give about nine per SIMD (1024 SIMDs), 16 at
+// most once the blocks alone are 128: more only adds partial slots for
+// k_assemble to read.  Below that a wavefront holds
+// a few omegas and a block's rows go to 48 to 64 wavefronts.  The
+// principal-value ladders take four lanes per omega once a lane's ladder is
+// shorter than what a wavefront waits for its slowest omega, and harmonic
+// blocks until the chip is full.  Device time of the three kernels with the
+// shapes before (8, 2 and 1 lanes from 2048, 8192 and 32768) and these, protons
+// and electrons on 128 x 256: 784 omegas 198 -> 141 us, 3192 537 -> 205,
+// 11990 1439 -> 330, 47961 1107 -> 693.
+LaunchShape pick_shape(int n, int rows) {
+  LaunchShape s;
+  if (n >= 1024) {
+    const int blocks = (n + 63) / 64;
+    const int tw = std::max(4, std::min((9216 + blocks - 1) / blocks, n >= 8192 ? 16 : 48));
+    const int w = n < 8192 ? 4 : 1;
+    s = {1, w, (tw + w - 1) / w, n >= 2048 ? 4 : 8, n >= 65536 ? 1 : (n >= 24576 ? 2 : 4)};
+  } else if (n >= 512) {
+    s = {4, 4, 12, 16, 8};
+  } else if (n >= 256) {
+    s = {8, 4, 16, 16, 8};
+  } else if (n >= 128) {
+    s = {16, 4, 12, 16, 8};
+  } else if (n >= 32) {
+    s = {16, 4, 16, 32, 8};
+  } else {
+    s = {64, 4, 16, 64, 8};
+  }
+  s.rc_a = std::max(1, std::min(s.rc_a, (rows + s.w_a - 1) / s.w_a));
+  return s;
 }
+
+bool shape_tuned(const alpsg_ctx *h, int n) { return h->tuned_valid[size_bucket(n)] != 0; }
 
 LaunchShape shape_for(const alpsg_ctx *h, int n) {
   const int b = size_bucket(n);
@@ -371,7 +402,9 @@ LaunchShape shape_for(const alpsg_ctx *h, int n) {
     const int *t = h->tuned_shape[b];
     return LaunchShape{t[0], t[1], t[2], t[3], t[4]};
   }
-  return pick_shape(n);
+  int rows = 0;
+  for (int s = 0; s < h->nspec; ++s) rows += std::max(h->prob.sp[s].nmax, 0) + 1;
+  return pick_shape(n, rows);
 }
 
 // the small-batch sweep (k_sweep_req<REQ_NCH, REQ_W, REQ_K> over REQ_TW / REQ_W
@@ -520,16 +553,26 @@ int alpsg_disp_on_scratch(alpsg_ctx *h, int n, const double *om, double *det,
   int dev = -1;
   HIPCHK(hipGetDevice(&dev));
   if (dev != h->device) return fail(ALPSG_E_STATE, "call on the device the handle was created on");
-  const LaunchShape sh = shape_for(h, n);
+  LaunchShape sh = shape_for(h, n);
   const int ns = h->nspec;
   const bool req = n <= REQ_MAX_N;
-  const size_t TW = req ? (size_t)REQ_TW : (size_t)sh.w_a * sh.rc_a;
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t b_om = up(sizeof(double2) * n), b_det = b_om;
-  const size_t b_a = up(sizeof(double2) * (size_t)n * TW * ns * 6);
-  const size_t b_b = up(sizeof(double2) * (size_t)n * ns * 2 * sh.rb * 6);
   const size_t b_z = req ? up(sizeof(int) * REQ_MAX_N) : 0;
-  const size_t need = b_om + b_det + b_a + b_b + b_z;
+  size_t b_a, b_b, need;
+  auto size_up = [&]() {
+    const size_t TW = req ? (size_t)REQ_TW : (size_t)sh.w_a * sh.rc_a;
+    b_a = up(sizeof(double2) * (size_t)n * TW * ns * 6);
+    b_b = up(sizeof(double2) * (size_t)n * ns * 2 * sh.rb * 6);
+    need = b_om + b_det + b_a + b_b + b_z;
+  };
+  size_up();
+  // a default shape whose partial slots do not fit gives way to the one of the
+  // fewest: four of the sweep, two of the resonant parts
+  if (need > scratch_bytes && !req && !shape_tuned(h, n)) {
+    sh = LaunchShape{1, 4, 1, 4, 1};
+    size_up();
+  }
   if (need > scratch_bytes)
     return fail(ALPSG_E_ARG, "batch of " + std::to_string(n) + " omegas needs " +
                                  std::to_string(need) + " bytes of scratch; the no-allocation path has " +

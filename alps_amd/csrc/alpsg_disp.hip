@@ -349,7 +349,10 @@ __device__ __forceinline__ void sweep_nodes_pf(cdptr srows, cdptr pa, int npar, 
   }
 }
 
-constexpr double SPLIT_MAX = 256.0;
+// the largest cancellation of G/m against C/den that the split form of a row is
+// used at: at 256 det D of the 256 x 256 map was 5e-14 from the 64-bit sums, at
+// 16 (7 % of that map's time more) it is 5e-15, as with the U r products
+constexpr double SPLIT_MAX = 16.0;
 constexpr int LPA = 1025;  // ppar points a sweep workgroup keeps in LDS (npar <= 1024)
 constexpr int LPA_REQ = 2056;  // the request sweep's: every species' grid at once up to this
 
@@ -1733,7 +1736,56 @@ __device__ __forceinline__ void assemble_block(
         for (int u = 0; u < 16; ++u) v = v + mk(buf[u].x, buf[u].y);
       }
     }
+    // chi_sk with the ee term and the normalisation; this thread also writes
+    // its mode's entries of the tensors (one thread per omega doing all of them
+    // took 60 us of a 45-omega batch)
+    const SpecDev &S = Pd.sp[s];
+    const double ee = Pd.kperp_norm ? S.int_ee : Pd.kperp * Pd.kperp * S.int_ee;
+    if (k == 2) v = v + mk(ee, 0.0);
+    const double norm = S.dens * S.q;
+    v = v * norm;
     lchi[t] = make_double2(v.re, v.im);
+    if (chi_out != nullptr || low_out != nullptr) {
+      const double2 ov = om_in[iom];
+      const cd om = mk(ov.x, ov.y);
+      cd dn = (om * om) * (Pd.vA * Pd.vA);
+      if (!Pd.kperp_norm) dn = dn * (Pd.kperp * Pd.kperp);
+      const int i = k < 3 ? k : (k == 5 ? 1 : 0), j = k < 3 ? k : (k == 3 ? 1 : 2);
+      const double sgn = k == 4 ? 1.0 : -1.0;  // the transposed entry's sign
+      if (chi_out != nullptr) {
+        double2 *o = chi_out + (size_t)iom * nspec * 9;
+        const cd c = cdiv(v, dn);
+        o[s + nspec * (i + 3 * j)] = make_double2(c.re, c.im);
+        if (i != j) o[s + nspec * (j + 3 * i)] = make_double2(sgn * c.re, sgn * c.im);
+      }
+      if (low_out != nullptr) {
+        double2 *o = low_out + (size_t)iom * nspec * 27;
+        for (int qq = 0; qq < 3; ++qq) {
+          cd tt = mk(0.0, 0.0);
+          const bool none = qq == 1 && (k == 0 || k == 3 || k == 4);
+          if (!none && S.rel) {
+            // relativistic: the parts k_rel_nonres, k_rel_res and k_rel_landau wrote; the
+            // ee term goes into chi only (ALPS_fns.f90:481-486)
+            for (int b = 0; b < LR; ++b) {
+              const double2 a = lowR[(((size_t)b * nom + iom) * nspec + s) * 18 + 6 * qq + k];
+              tt = tt + mk(a.x, a.y);
+            }
+          } else if (!none) {
+            const double2 a = lowA[((size_t)iom * nspec + s) * 18 + 6 * qq + k];
+            tt = mk(a.x, a.y);
+            for (int b = 0; b < 2 * RB; ++b) {
+              const double2 u = lowB[(((size_t)iom * nspec + s) * (2 * RB) + b) * 18 + 6 * qq + k];
+              tt = tt + mk(u.x, u.y);
+            }
+            if (qq == 1 && k == 2) tt = tt + mk(ee, 0.0);
+          }
+          const cd c = none ? mk(0.0, 0.0) : cdiv(tt * norm, dn);
+          o[s + nspec * (i + 3 * (j + 3 * qq))] = make_double2(c.re, c.im);
+          if (i != j)
+            o[s + nspec * (j + 3 * (i + 3 * qq))] = make_double2(sgn * c.re, sgn * c.im);
+        }
+      }
+    }
   }
   __syncthreads();
   if (!in || sk != 0) return;
@@ -1741,69 +1793,11 @@ __device__ __forceinline__ void assemble_block(
   const cd om = mk(ov.x, ov.y);
   cd eps[6];
   for (int q = 0; q < 6; ++q) eps[q] = mk(0.0, 0.0);
-  cd dn = (om * om) * (Pd.vA * Pd.vA);
-  if (!Pd.kperp_norm) dn = dn * (Pd.kperp * Pd.kperp);
-  for (int sp = 0; sp < nspec; ++sp) {
-    const SpecDev &S = Pd.sp[sp];
-    cd chi[6];
+  for (int sp = 0; sp < nspec; ++sp)
     for (int q = 0; q < 6; ++q) {
       const double2 a = lchi[lo_om * per + sp * 6 + q];
-      chi[q] = mk(a.x, a.y);
+      eps[q] = eps[q] + mk(a.x, a.y);
     }
-    const double ee = Pd.kperp_norm ? S.int_ee : Pd.kperp * Pd.kperp * S.int_ee;
-    chi[2] = chi[2] + mk(ee, 0.0);
-    const double norm = S.dens * S.q;
-    for (int q = 0; q < 6; ++q) {
-      chi[q] = chi[q] * norm;
-      eps[q] = eps[q] + chi[q];
-    }
-    if (chi_out != nullptr) {
-      double2 *o = chi_out + (size_t)iom * nspec * 9;
-      cd v[3][3];
-      for (int q = 0; q < 6; ++q) v[MI[q]][MJ[q]] = cdiv(chi[q], dn);
-      v[1][0] = mk(-v[0][1].re, -v[0][1].im);
-      v[2][0] = v[0][2];
-      v[2][1] = mk(-v[1][2].re, -v[1][2].im);
-      for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 3; ++j) o[sp + nspec * (i + 3 * j)] = make_double2(v[i][j].re, v[i][j].im);
-    }
-    if (low_out != nullptr) {
-      double2 *o = low_out + (size_t)iom * nspec * 27;
-      for (int qq = 0; qq < 3; ++qq) {
-        cd v[3][3];
-        for (int i = 0; i < 3; ++i)
-          for (int j = 0; j < 3; ++j) v[i][j] = mk(0.0, 0.0);
-        for (int q = 0; q < 6; ++q) {
-          if (qq == 1 && (q == 0 || q == 3 || q == 4)) continue;
-          cd tt;
-          if (S.rel) {
-            // relativistic: the parts k_rel_nonres, k_rel_res and k_rel_landau wrote; the
-            // ee term goes into chi only (ALPS_fns.f90:481-486)
-            tt = mk(0.0, 0.0);
-            for (int j = 0; j < LR; ++j) {
-              const double2 a = lowR[(((size_t)j * nom + iom) * nspec + sp) * 18 + 6 * qq + q];
-              tt = tt + mk(a.x, a.y);
-            }
-          } else {
-            const double2 a = lowA[((size_t)iom * nspec + sp) * 18 + 6 * qq + q];
-            tt = mk(a.x, a.y);
-            for (int b = 0; b < 2 * RB; ++b) {
-              const double2 u = lowB[(((size_t)iom * nspec + sp) * (2 * RB) + b) * 18 + 6 * qq + q];
-              tt = tt + mk(u.x, u.y);
-            }
-            if (qq == 1 && q == 2) tt = tt + mk(ee, 0.0);
-          }
-          v[MI[q]][MJ[q]] = cdiv(tt * norm, dn);
-        }
-        v[1][0] = mk(-v[0][1].re, -v[0][1].im);
-        v[2][0] = v[0][2];
-        v[2][1] = mk(-v[1][2].re, -v[1][2].im);
-        for (int i = 0; i < 3; ++i)
-          for (int j = 0; j < 3; ++j)
-            o[sp + nspec * (i + 3 * (j + 3 * qq))] = make_double2(v[i][j].re, v[i][j].im);
-      }
-    }
-  }
   // dielectric tensor, wave tensor, determinant (ALPS_fns.f90:566-624)
   const cd unit = Pd.kperp_norm ? (om * Pd.vA) * (om * Pd.vA)
                                 : ((Pd.kperp * om) * Pd.vA) * ((Pd.kperp * om) * Pd.vA);
