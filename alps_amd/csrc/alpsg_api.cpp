@@ -49,7 +49,8 @@ hipError_t launch_sweep_req(hipStream_t st, int nch, int W, int RC, int K, const
                             bool reduce);
 hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec, int nom,
                            const double2 *om, const int *active, double2 *chiB, double2 *lowB,
-                           int lgen, const int *pidx = nullptr, int P = 0);
+                           int lgen, const int *pidx = nullptr, int P = 0,
+                           const LandTabs *tabs = nullptr);
 hipError_t launch_nhds(hipStream_t st, const ProbDev *prob, int nspec, int nom, const double2 *om,
                        const int *active, double2 *chiA, double2 *lowA, const int *pidx = nullptr);
 int nhds_tables(double z, int bm_nmax, double bessel_zero, std::vector<double2> &tab);
@@ -83,6 +84,8 @@ hipError_t launch_rel(hipStream_t st, const ProbDev *prob, int nspec, int nmaxR,
 RelSplit rel_split(int nom);
 int rel_slots(RelSplit sp, int nmaxR);
 int rel_low_slots(RelSplit sp);
+hipError_t launch_land_build(hipStream_t st, const ProbDev *prob, int nspec, int ny, int nr,
+                             const LandTabs &T);
 hipError_t launch_assemble(hipStream_t st, const ProbDev *prob, int nspec, int nom, int W, int RB,
                            const double2 *om, const int *active, const double2 *chiA,
                            const double2 *chiB, const double2 *lowA, const double2 *lowB,
@@ -246,6 +249,10 @@ struct alpsg_ctx {
   // Landau forms the species take: bit 0 a call of eval_fit, bit 1 the inlined
   // kappa evaluation (species whose every fit is a kappa fit)
   int lgen = 0;
+  // Landau tables of the current batch (alpsg_land.hip)
+  DevBuf<double> landc[ALPSG_MAXSPEC];
+  DevBuf<unsigned char> landok[ALPSG_MAXSPEC], landneed;
+  DevBuf<int> landcut;
   // closed-form (use_bM) species and their &bM_spec parameters
   int usebm[ALPSG_MAXSPEC] = {0};
   bool any_bm = false;
@@ -305,7 +312,11 @@ struct alpsg_ctx {
       gampp[s].release();
       dfrel[s].release();
       rowlim[s].release();
+      landc[s].release();
+      landok[s].release();
     }
+    landneed.release();
+    landcut.release();
     mtab.release();
     prob_d.release();
     om_d.release();
@@ -435,7 +446,8 @@ struct DispBufs {
 // (sized by the caller; nothing is allocated here).  Relativistic species take
 // the handle's own buffers, so callers with B outside the handle exclude them.
 int disp_chain(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_dev,
-               const DispBufs &B, bool want_chi, bool want_low, bool want_wave, LaunchShape sh) {
+               const DispBufs &B, bool want_chi, bool want_low, bool want_wave, LaunchShape sh,
+               const LandTabs *tabs = nullptr) {
   const int ns = h->nspec;
   const int TW = sh.w_a * sh.rc_a;
   // Small batches (a few roots' secant steps, the one-omega plain path): the
@@ -457,7 +469,7 @@ int disp_chain(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_dev
                                h->lgen));
   else
     HIPCHK(launch_resonant(h->st, sh.nch_b, sh.rb, h->prob_d.p, ns, n, om_dev, active_dev, B.chiB,
-                           want_low ? B.lowB : nullptr, h->lgen, nullptr, h->P));
+                           want_low ? B.lowB : nullptr, h->lgen, nullptr, h->P, tabs));
   if (h->any_bm)
     HIPCHK(launch_nhds(h->st, h->prob_d.p, ns, n, om_dev, active_dev, B.chiA,
                        want_low ? B.lowA : nullptr));
@@ -507,9 +519,94 @@ int ensure_series(alpsg_ctx *h, int n) {
   return ALPSG_OK;
 }
 
+// The frequencies of a batch, as far as the host knows them.
+struct OmBounds {
+  double re_lo = 0.0, re_hi = -1.0, im_lo = 0.0;  // re_hi < re_lo: unknown
+};
+
+OmBounds bounds_of(const double *om, int n) {
+  OmBounds b;
+  b.re_lo = b.re_hi = om[0];
+  b.im_lo = om[1];
+  for (int i = 1; i < n; ++i) {
+    b.re_lo = std::min(b.re_lo, om[2 * i]);
+    b.re_hi = std::max(b.re_hi, om[2 * i]);
+    b.im_lo = std::min(b.im_lo, om[2 * i + 1]);
+  }
+  return b;
+}
+
+// The Landau tables of a batch (alpsg_land.hip) for the kappa species, built on
+// the handle's stream; use false, with nothing built, where no species gains.  A
+// tile takes LT_N evaluations per pperp row where the batch's row sums take one
+// per omega and resonant harmonic; with the transform and the launch a tile costs
+// about twice its evaluations, so the tables are built from 64 row sums per tile
+// on.  A Chebyshev continuation's row sums cost a third of a kappa fit's, and most
+// of its tiles are clipped (96 x 64 omegas: 99 us of row sums, 250 us of tables),
+// so it keeps them.
+constexpr int LAND_MIN = 512;
+
+int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, int RB, LandTabs &T, bool &use) {
+  use = false;
+  if (n < LAND_MIN || (h->lgen & 2) == 0 || !(b.re_lo <= b.re_hi) || !std::isfinite(b.re_lo) ||
+      !std::isfinite(b.re_hi) || !std::isfinite(b.im_lo) || b.im_lo > 0.0)
+    return ALPSG_OK;
+  const double kpar = h->prob.kpar;
+  std::memset(&T, 0, sizeof(T));
+  int ny_max = 0, nr_max = 0;
+  for (int s = 0; s < h->nspec; ++s) {
+    const SpecDev &S = h->prob.sp[s];
+    if (!S.fit_kappa || h->relsp[s] || h->usebm[s] || S.nmax < 0) continue;
+    const double *pa = &h->ppar_h[(size_t)s * (h->npar + 1)];
+    // the resonant momenta determine_resonances accepts
+    const double L = pa[1] - h->P * S.dppar;
+    const double U = std::max(pa[h->npar], pa[h->npar - 1] + h->P * S.dppar);
+    // (a little wider: an edge momentum may round past the last tile; few bits, so
+    // the centres' imaginary parts are exact)
+    const double t = (double)(float)((U - L) * (1.0 + 1e-6) / LT_NX);
+    const double depth = -h->ms[s] * b.im_lo / std::fabs(kpar);
+    const double ny = std::floor(depth / t) + 1.0;
+    // a resonance needs m Re om - kpar p = n q within the grid
+    const double q = std::fabs(h->qs[s]);
+    const double e = std::max(std::fabs(h->ms[s] * b.re_lo), std::fabs(h->ms[s] * b.re_hi)) +
+                     std::fabs(kpar) * std::max(std::fabs(L), std::fabs(U));
+    const int nr = (int)std::min((double)S.nmax, std::ceil(e / q) + 1.0);
+    const double rows = std::fabs(kpar) * (U - L) / q;  // resonant harmonics of an omega
+    if (!(t > 0.0) || !(ny <= LT_NY) || nr > LT_NR || (double)n * rows < 64.0 * LT_NX * ny) continue;
+    LandTab &tb = T.sp[s];
+    tb.ny = (int)ny;
+    tb.nr = nr;
+    tb.x0 = L;
+    tb.t = t;
+    tb.it = 1.0 / t;
+    tb.ir = std::sqrt(2.0) / t;
+    const size_t tiles = (size_t)LT_NX * tb.ny + LT_MAXP * LT_SUB * LT_SUB;
+    if (h->landcut.ensure((size_t)ALPSG_MAXSPEC * LT_MAXP) != hipSuccess ||
+        h->landc[s].ensure(tiles * (nr + 1) * 3 * LT_J * 4) != hipSuccess ||
+        h->landok[s].ensure(tiles) != hipSuccess ||
+        h->landneed.ensure((size_t)h->nspec * RB * n) != hipSuccess) {
+      (void)hipGetLastError();  // no room: the row sums need none
+      continue;
+    }
+    tb.cut = h->landcut.p + s * LT_MAXP;
+    tb.c = h->landc[s].p;
+    tb.ok = h->landok[s].p;
+    ny_max = std::max(ny_max, tb.ny);
+    nr_max = std::max(nr_max, nr);
+    use = true;
+  }
+  if (!use) return ALPSG_OK;
+  T.need = h->landneed.p;
+  HIPCHK(launch_land_build(h->st, h->prob_d.p, h->nspec, ny_max, nr_max, T));
+  return ALPSG_OK;
+}
+
 int disp_device(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_dev, bool want_chi,
-                bool want_low, bool want_wave, LaunchShape sh) {
+                bool want_low, bool want_wave, LaunchShape sh, const OmBounds &ob = OmBounds()) {
   if (const int rc = ensure_series(h, n)) return rc;
+  LandTabs tabs;
+  bool use_tabs = false;
+  if (const int rc = landau_tables(h, n, ob, sh.rb, tabs, use_tabs)) return rc;
   const int ns = h->nspec;
   const int TW = sh.w_a * sh.rc_a;
   HIPCHK(h->det_d.ensure(n));
@@ -532,7 +629,8 @@ int disp_device(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_de
   }
   DispBufs B{h->det_d.p, h->chiA_d.p, h->chiB_d.p, h->chi_d.p, h->low_d.p, h->lowA_d.p,
              h->lowB_d.p, h->wave_d.p, h->zidx.p};
-  return disp_chain(h, n, om_dev, active_dev, B, want_chi, want_low, want_wave, sh);
+  return disp_chain(h, n, om_dev, active_dev, B, want_chi, want_low, want_wave, sh,
+                    use_tabs ? &tabs : nullptr);
 }
 
 }  // namespace
@@ -637,6 +735,7 @@ int autotune(alpsg_ctx *h, int n, const double2 *om_host, int *shape_out) {
     best = tot / 2;
     return ALPSG_OK;
   };
+  const OmBounds ob = bounds_of(reinterpret_cast<const double *>(om.data()), n);
   std::vector<std::pair<float, LaunchShape>> candA, candB;
   const int rcs[] = {1, 2, 3, 4, 6, 8, 12, 16};
   for (auto &v : kSweepVariants) {
@@ -664,11 +763,15 @@ int autotune(alpsg_ctx *h, int n, const double2 *om_host, int *shape_out) {
     for (int rb : rbs) {
       if ((size_t)n * ns * 2 * rb * 6 * sizeof(double2) > budget) continue;
       HIPCHK(h->chiB_d.ensure((size_t)n * ns * 2 * rb * 6));
+      LandTabs tabs;
+      bool ut = false;
+      if (const int rc = landau_tables(h, n, ob, rb, tabs, ut)) return rc;
       float t;
       int rc_ = time_launch(
           [&]() {
             return launch_resonant(h->st, nb, rb, h->prob_d.p, ns, n, h->om_d.p, nullptr,
-                                   h->chiB_d.p, nullptr, h->lgen, nullptr, h->P);
+                                   h->chiB_d.p, nullptr, h->lgen, nullptr, h->P,
+                                   ut ? &tabs : nullptr);
           },
           t);
       if (rc_) return rc_;
@@ -692,7 +795,7 @@ int autotune(alpsg_ctx *h, int n, const double2 *om_host, int *shape_out) {
       float t;
       int rc_ = time_launch(
           [&]() -> hipError_t {
-            return disp_device(h, n, h->om_d.p, nullptr, false, false, false, sh) == ALPSG_OK
+            return disp_device(h, n, h->om_d.p, nullptr, false, false, false, sh, ob) == ALPSG_OK
                        ? hipSuccess
                        : hipErrorUnknown;
           },
@@ -806,7 +909,9 @@ int run_disp(alpsg_ctx *h, int n, const double *om, double *det, double *chi, do
   }
   LaunchShape sh = shape_for(h, n);
   HIPCHK(hipEventRecord(h->ev0, h->st));
-  int rc = disp_device(h, n, h->om_d.p, nullptr, chi != nullptr, low != nullptr, wave != nullptr, sh);
+  const OmBounds ob = n >= LAND_MIN && h->lgen ? bounds_of(om, n) : OmBounds();
+  int rc = disp_device(h, n, h->om_d.p, nullptr, chi != nullptr, low != nullptr, wave != nullptr, sh,
+                       ob);
   if (rc) return rc;
   HIPCHK(hipEventRecord(h->ev1, h->st));
   HIPCHK(hipMemcpyAsync(pin ? (void *)h->det_pin.p : (void *)det, h->det_d.p, sizeof(double2) * n,
@@ -2426,7 +2531,11 @@ int map_search_core(alpsg_ctx *h, double omi, double omf, double gami, double ga
   }
   LaunchShape sh = shape_for(h, (int)N);
   HIPCHK(hipEventRecord(h->ev0, h->st));
-  int rc = disp_device(h, (int)N, h->om_d.p, nullptr, false, false, false, sh);
+  OmBounds ob;
+  ob.re_lo = std::min(omi, omf);
+  ob.re_hi = std::max(omi, omf);
+  ob.im_lo = std::min(gami, gamf);
+  int rc = disp_device(h, (int)N, h->om_d.p, nullptr, false, false, false, sh, ob);
   if (rc) return rc;
   HIPCHK(hipEventRecord(h->ev1, h->st));
   HIPCHK(h->mcal_d.ensure(N));

@@ -111,6 +111,29 @@ struct RelSplit {
   int B, RS;
 };
 
+// Landau tables of a batch (alpsg_land.hip): square tiles of side t over Re p in
+// [x0, x0 + LT_NX t], Im p in [-ny t, 0], LT_J Taylor coefficients per tile
+#define LT_N 32   // points of a tile's circle
+#define LT_J 24   // coefficients used
+#define LT_NX 64  // tiles across
+#define LT_NY 24  // tile rows at most
+#define LT_NR 9   // harmonics 0..LT_NR at most
+#define LT_SUB 4  // a tile whose series does not converge is cut into LT_SUB^2 smaller ones,
+#define LT_MAXP 48  // this many tiles at most
+struct LandTab {
+  // tiles: LT_NX ny of side t, then LT_SUB^2 small ones of each of the LT_MAXP cut
+  double *c;          // [tile][n 0..nr][a 0..2][LT_J]{A re, im, B re, im}, NULL: no table
+  unsigned char *ok;  // [tile]: 0 not usable, 1 series, 2 + i: the i-th tile cut
+  int *cut;           // [LT_MAXP]: the tiles cut, -1 past the last
+  int ny, nr;
+  double x0, t, it, ir;  // it = 1/t; ir = 1/(half diagonal of a tile)
+};
+struct LandTabs {
+  LandTab sp[ALPSG_DMAXSPEC];
+  // [species][harmonic block][omega]: a row of this omega is left to the row sums
+  unsigned char *need;
+};
+
 // ---------------------------------------------------------------------------
 // Small complex helpers (double2 = (re, im)).
 // ---------------------------------------------------------------------------

@@ -1465,6 +1465,62 @@ __device__ void landau_part(const SpecDev &S, const ProbDev &Pd, int an, const R
 
 }  // namespace
 
+namespace {
+
+// harmonics nlo..nhi whose p_res = (m w - n q)/kpar can satisfy determine_resonances:
+// Re p_res in [pa[1] - P dppar, max(pa[npar], pa[npar-1] + P dppar)), widened by one
+__device__ __forceinline__ void res_harmonics(const SpecDev &S, int P, double kpar, double omr,
+                                              bool valid, int &nlo, int &nhi) {
+  nlo = 1;
+  nhi = 0;
+  if (!valid || omr != omr) return;
+  const double L = S.ppar[1] - P * S.dppar;
+  const double U = fmax(S.ppar[S.npar], S.ppar[S.npar - 1] + P * S.dppar);
+  const double n1 = (S.m * omr - kpar * L) / S.q, n2 = (S.m * omr - kpar * U) / S.q;
+  const double lo_d = fmin(n1, n2) - 1.0, hi_d = fmax(n1, n2) + 1.0;
+  nlo = (int)fmax(floor(lo_d), -(double)S.nmax);
+  nhi = (int)fmin(ceil(hi_d), (double)S.nmax);
+}
+
+// the modes of harmonic n's Landau term from its pperp sums (int_T_res,
+// ALPS_fns.f90:1768-1808): zz, xz, yz take p_res
+__device__ __forceinline__ void landau_modes(const ProbDev &Pd, const SpecDev &S, int n,
+                                             const RowClass &rc, cd Ls0, cd Ls1, cd Ls2,
+                                             cd add[6]) {
+  const cd p = mk(rc.pr, rc.pim);
+  const cd Lm[6] = {Ls0, Ls1, Ls0 * (p * p), Ls2, Ls0 * p, Ls2 * p};
+  const double f = -(double)rc.landau * S.dpperp * PI_D * 2.0 * PI_D;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) add[k] = timesI(f * (Lm[k] * tconst(Pd, S, n, k)));
+  if (n == 0) add[0] = add[3] = add[4] = mk(0.0, 0.0);
+}
+
+// the usable tile of the Landau tables that holds (pr, pim), -1 if none; (zr, zi):
+// the place in it, in half diagonals from its centre
+__device__ __forceinline__ int land_tile(const LandTab &T, int an, double pr, double pim,
+                                         double &zr, double &zi) {
+  const double x = (pr - T.x0) * T.it, y = -pim * T.it;
+  zr = zi = 0.0;
+  if (!(an <= T.nr && x >= 0.0 && x < (double)LT_NX && y >= 0.0 && y < (double)T.ny)) return -1;
+  const int ix = (int)x, iy = (int)y;
+  int tile = iy * LT_NX + ix;
+  const int st = T.ok[tile];
+  // from the centre itself, as k_land_build rounds it: the place to the last bit
+  if (st < 2) {
+    zr = (pr - __builtin_fma(ix + 0.5, T.t, T.x0)) * T.ir;
+    zi = (pim + (iy + 0.5) * T.t) * T.ir;
+    return st == 0 ? -1 : tile;
+  }
+  const int iu = min((int)((x - ix) * LT_SUB), LT_SUB - 1);
+  const int iv = min((int)((y - iy) * LT_SUB), LT_SUB - 1);
+  tile = LT_NX * T.ny + (st - 2) * (LT_SUB * LT_SUB) + iv * LT_SUB + iu;
+  zr = (pr - __builtin_fma(ix + (iu + 0.5) / LT_SUB, T.t, T.x0)) * (LT_SUB * T.ir);
+  zi = (pim + (iy + (iv + 0.5) / LT_SUB) * T.t) * (LT_SUB * T.ir);
+  return T.ok[tile] == 0 ? -1 : tile;
+}
+
+}  // namespace
+
 // PART 0: principal-value terms; PART 1: Landau terms of species whose analytic
 // continuation is one Maxwellian with pperp-independent (u2, u3); PART 3: Landau
 // terms of species whose every fit is a kappa fit; PART 2: Landau terms of the
@@ -1480,7 +1536,8 @@ __device__ __forceinline__ void resonant_body(const ProbDev *__restrict__ probp,
                                               double2 *__restrict__ lowB,
                                               const int *__restrict__ pidx, int RB, int rb, int bx,
                                               int by, int lane, double *win_lds,
-                                              int pvw = PV_WIN) {
+                                              int pvw = PV_WIN, LandTab tab = LandTab{},
+                                              const unsigned char *tab_need = nullptr) {
   constexpr int OMB = 64 / NCH;
   const ProbDev &Pd = (NCH == 64 && pidx != nullptr) ? probp[pidx[bx]] : *probp;
   const int g = lane / NCH, c = lane % NCH;
@@ -1498,32 +1555,35 @@ __device__ __forceinline__ void resonant_body(const ProbDev *__restrict__ probp,
   const bool kap_s = S.fit_kappa != 0;
   if ((PART == 1 && !uni_s) || (PART == 2 && (uni_s || kap_s)) || (PART == 3 && !kap_s)) return;
   double *win = win_lds + g * (2 * pvw);  // pvw >= 2P + 8, the window's extent
+  // a species with Landau tables: k_resonant_tab has written this slot, and only
+  // the rows its tiles do not cover are added here
+  const bool tabbed = PART == 3 && tab.c != nullptr;
+  bool left = false;
+  if (tabbed) {
+    left = valid && tab_need[((size_t)s * RB + rb) * nom + iom] != 0;
+    if (!__any(left)) return;
+  }
   cd res[6];
 #pragma unroll
   for (int k = 0; k < 6; ++k) res[k] = mk(0.0, 0.0);
   double2 *lo = (lowB != nullptr && valid && c == 0)
                     ? lowB + (((size_t)iom * nspec + s) * (2 * RB) + slot) * 18
                     : nullptr;
-  if (lo)
+  if (lo && !tabbed)
     for (int t = 0; t < 18; ++t) lo[t] = make_double2(0.0, 0.0);
 
-  // harmonics whose p_res = (m w - n q)/kpar can satisfy determine_resonances:
-  // Re p_res in [pa[1] - P dppar, max(pa[npar], pa[npar-1] + P dppar)), widened by one
-  int nlo = 1, nhi = 0;
-  if (valid && omr == omr) {
-    const double L = S.ppar[1] - P * S.dppar;
-    const double U = fmax(S.ppar[npar], S.ppar[npar - 1] + P * S.dppar);
-    const double n1 = (S.m * omr - kpar * L) / S.q, n2 = (S.m * omr - kpar * U) / S.q;
-    const double lo_d = fmin(n1, n2) - 1.0, hi_d = fmax(n1, n2) + 1.0;
-    nlo = (int)fmax(floor(lo_d), -(double)S.nmax);
-    nhi = (int)fmin(ceil(hi_d), (double)S.nmax);
-  }
+  int nlo, nhi;
+  res_harmonics(S, P, kpar, omr, valid, nlo, nhi);
   const double scaleN = 2.0 * PI_D * S.dpperp * 0.25 * (-S.q / kpar);
   for (int n = nlo + rb; n <= nhi; n += RB) {
     RowClass rc;
     classify(S, P, kpar, omr, omi, n, rc, (gdptr)S.ppar);
     if (!rc.found || (PART == 0 && !rc.pv) || (PART != 0 && !rc.landau)) continue;
     const int an = n < 0 ? -n : n;
+    if (tabbed) {
+      double zr, zi;
+      if (!left || land_tile(tab, an, rc.pr, rc.pim, zr, zi) >= 0) continue;
+    }
     const double *rows = S.nodes + (size_t)an * (npar - 1) * NODE_STRIDE;
     cd add[6];
 #pragma unroll
@@ -1564,13 +1624,7 @@ __device__ __forceinline__ void resonant_body(const ProbDev *__restrict__ probp,
                                                                              omi, c, L, zero);
       zero = gor<NCH>(zero);
       if (!zero) {
-        const cd p = mk(rc.pr, rc.pim);
-        const cd Ls0 = gsumc<NCH>(L[0]), Ls1 = gsumc<NCH>(L[1]), Ls2 = gsumc<NCH>(L[2]);
-        // T_res (int_T_res, ALPS_fns.f90:1768-1808): zz, xz, yz take p_res
-        const cd Lm[6] = {Ls0, Ls1, Ls0 * (p * p), Ls2, Ls0 * p, Ls2 * p};
-        const double f = -(double)rc.landau * S.dpperp * PI_D * 2.0 * PI_D;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) add[k] = add[k] + timesI(f * (Lm[k] * tconst(Pd, S, n, k)));
+        landau_modes(Pd, S, n, rc, gsumc<NCH>(L[0]), gsumc<NCH>(L[1]), gsumc<NCH>(L[2]), add);
       }
     }
     if (n == 0) {
@@ -1585,6 +1639,92 @@ __device__ __forceinline__ void resonant_body(const ProbDev *__restrict__ probp,
   }
   if (valid && c == 0) {
     // omega-fastest layout: chiB[((slot * nspec + s) * 6 + k) * nom + iom]
+    double2 *o = chiB + ((size_t)(slot * nspec + s) * 6) * nom + iom;
+    if (tabbed) {
+      if (left)
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          const double2 a = o[(size_t)k * nom];
+          o[(size_t)k * nom] = make_double2(a.x + res[k].re, a.y + res[k].im);
+        }
+      return;
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) o[(size_t)k * nom] = make_double2(res[k].re, res[k].im);
+  }
+}
+
+// The Landau part from the tables: four lanes per omega, lane a < 3 of them
+// sums the Taylor series of A_a + n B_a; grid (omega blocks of 16, species, RB).
+// Rows outside the usable tiles set need for the launch of the row sums that
+// follows.  On a 512 x 512 map of a kappa core and beam (256 x 512 grid) the
+// Landau pass takes 1.4 ms with the tables' build against 13.6 ms of row sums.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_resonant_tab(
+    const ProbDev *__restrict__ probp, int nom, const double2 *__restrict__ om_in,
+    const int *__restrict__ active, double2 *__restrict__ chiB, double2 *__restrict__ lowB,
+    LandTabs tabs) {
+  const int lane = threadIdx.x, g = lane >> 2, c = lane & 3;
+  const int s = blockIdx.y, RB = gridDim.z, rb = blockIdx.z, slot = RB + rb;
+  const LandTab &T = tabs.sp[s];
+  if (T.c == nullptr) return;
+  const ProbDev &Pd = *probp;
+  const int iom = blockIdx.x * 16 + g;
+  const bool valid = (iom < nom) && (active == nullptr || active[iom] != 0);
+  const double2 ov = valid ? om_in[iom] : make_double2(1.0, 0.5);
+  const double omr = ov.x, omi = ov.y;
+  const int nspec = Pd.nspec;
+  const SpecDev &S = Pd.sp[s];
+  const int P = Pd.P;
+  const double kpar = Pd.kpar;
+  cd res[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) res[k] = mk(0.0, 0.0);
+  double2 *lo = (lowB != nullptr && valid && c == 0)
+                    ? lowB + (((size_t)iom * nspec + s) * (2 * RB) + slot) * 18
+                    : nullptr;
+  if (lo)
+    for (int t = 0; t < 18; ++t) lo[t] = make_double2(0.0, 0.0);
+  int nlo, nhi;
+  res_harmonics(S, P, kpar, omr, valid, nlo, nhi);
+  int need = 0;
+  for (int n = nlo + rb; n <= nhi; n += RB) {
+    RowClass rc;
+    classify(S, P, kpar, omr, omi, n, rc, (gdptr)S.ppar);
+    if (!rc.found || !rc.landau) continue;
+    const int an = n < 0 ? -n : n;
+    double zr, zi;
+    const int tile = land_tile(T, an, rc.pr, rc.pim, zr, zi);
+    if (tile < 0) {
+      need = 1;
+      continue;
+    }
+    const double4 *cf = reinterpret_cast<const double4 *>(T.c) +
+                        (((size_t)tile * (T.nr + 1) + an) * 3 + min(c, 2)) * LT_J;
+    const double dn = (double)n;
+    cd L = mk(0.0, 0.0);
+#pragma unroll 8
+    for (int j = LT_J - 1; j >= 0; --j) {
+      const double4 v = cf[j];
+      const double cr = __builtin_fma(dn, v.z, v.x), ci = __builtin_fma(dn, v.w, v.y);
+      const double re = __builtin_fma(L.re, zr, __builtin_fma(-L.im, zi, cr));
+      L.im = __builtin_fma(L.re, zi, __builtin_fma(L.im, zr, ci));
+      L.re = re;
+    }
+    const int l0 = lane & ~3;
+    const cd Ls0 = mk(__shfl(L.re, l0, 64), __shfl(L.im, l0, 64));
+    const cd Ls1 = mk(__shfl(L.re, l0 + 1, 64), __shfl(L.im, l0 + 1, 64));
+    const cd Ls2 = mk(__shfl(L.re, l0 + 2, 64), __shfl(L.im, l0 + 2, 64));
+    cd add[6];
+    landau_modes(Pd, S, n, rc, Ls0, Ls1, Ls2, add);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) res[k] = res[k] + add[k];
+    if (lo && an <= 1) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) lo[6 * (n + 1) + k] = make_double2(add[k].re, add[k].im);
+    }
+  }
+  if (valid && c == 0) {
+    tabs.need[((size_t)s * RB + rb) * nom + iom] = (unsigned char)need;
     double2 *o = chiB + ((size_t)(slot * nspec + s) * 6) * nom + iom;
 #pragma unroll
     for (int k = 0; k < 6; ++k) o[(size_t)k * nom] = make_double2(res[k].re, res[k].im);
@@ -1630,10 +1770,10 @@ template <int NCH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_resonant_kappa(
     const ProbDev *__restrict__ probp, int nom, const double2 *__restrict__ om_in,
     const int *__restrict__ active, double2 *__restrict__ chiB, double2 *__restrict__ lowB,
-    const int *__restrict__ pidx) {
-  __shared__ double win[(64 / NCH) * 2 * PV_WIN];
+    const int *__restrict__ pidx, bool use_tabs, LandTabs tabs) {
   resonant_body<NCH, 3>(probp, nom, om_in, active, chiB, lowB, pidx, gridDim.z, blockIdx.z,
-                        blockIdx.x, blockIdx.y, threadIdx.x, win);
+                        blockIdx.x, blockIdx.y, threadIdx.x, nullptr, PV_WIN,
+                        use_tabs ? tabs.sp[blockIdx.y] : LandTab{}, tabs.need);
 }
 
 // The principal-value and Landau parts in one launch (small batches, where a
@@ -1903,10 +2043,19 @@ hipError_t launch_sweep_req(hipStream_t st, int nch, int W, int RC, int K, const
 // the launch (<= 0: unknown, the largest window)
 hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec, int nom,
                            const double2 *om, const int *active, double2 *chiB, double2 *lowB,
-                           int lgen, const int *pidx, int P) {
+                           int lgen, const int *pidx, int P, const LandTabs *tabs) {
   if (nom <= 0) return hipSuccess;
-  if (pidx != nullptr && nch != 64) return hipErrorInvalidValue;
+  if (pidx != nullptr && (nch != 64 || tabs != nullptr)) return hipErrorInvalidValue;
+  const LandTabs tb = tabs != nullptr ? *tabs : LandTabs{};
+  const bool ut = tabs != nullptr;
+  // (the rows left to the row sums are few: many lanes each, and a wavefront
+  // without any ends at once)
+  const int nchl = !ut ? nch : (nom <= 16384 ? 64 : 16);
+  if (ut)
+    hipLaunchKernelGGL(k_resonant_tab, dim3((nom + 15) / 16, nspec, RB), dim3(64), 0, st, prob, nom,
+                       om, active, chiB, lowB, tb);
   const int pvw = (P >= 1 && 2 * P + 8 <= PV_WIN) ? 2 * P + 8 : PV_WIN;
+  bool done = false;
 #define RS(N)                                                                                  \
   if (nch == N) {                                                                              \
     const int grid = (nom + (64 / N) - 1) / (64 / N);                                          \
@@ -1918,14 +2067,20 @@ hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob,
     if (lgen & 1)                                                                              \
       hipLaunchKernelGGL((k_resonant_gen<N>), dim3(grid, nspec, RB), dim3(64), 0, st, prob, nom, \
                          om, active, chiB, lowB, pidx, pvw);                                   \
-    if (lgen & 2)                                                                              \
-      hipLaunchKernelGGL((k_resonant_kappa<N>), dim3(grid, nspec, RB), dim3(64), 0, st, prob,   \
-                         nom, om, active, chiB, lowB, pidx);                                   \
-    return hipGetLastError();                                                                  \
+    done = true;                                                                               \
   }
   RS(4) RS(8) RS(16) RS(32) RS(64)
 #undef RS
-  return hipErrorInvalidValue;
+  if (!done) return hipErrorInvalidValue;
+#define RL(N)                                                                                  \
+  if (nchl == N)                                                                               \
+    hipLaunchKernelGGL((k_resonant_kappa<N>), dim3((nom + (64 / N) - 1) / (64 / N), nspec, RB), \
+                       dim3(64), 0, st, prob, nom, om, active, chiB, lowB, pidx, ut, tb);
+  if (lgen & 2) {
+    RL(4) RL(8) RL(16) RL(32) RL(64)
+  }
+#undef RL
+  return hipGetLastError();
 }
 
 hipError_t launch_assemble(hipStream_t st, const ProbDev *prob, int nspec, int nom, int W, int RB,
