@@ -37,10 +37,7 @@ hipError_t launch_int_ee(hipStream_t st, int nspec, int nperp, int npar, const d
                          const double *qs, const double *ms, double *out);
 hipError_t launch_bessel_max(hipStream_t st, int nspec, int nperp, int ntry, double kperp,
                              const double *pperp, const double *qs, const int *mtab, double *out);
-hipError_t launch_species_k(hipStream_t st, int nperp, int npar, int nmax, double kperp,
-                            double kpar, double q, double m, const double *pperp,
-                            const double *ppar, const double *df1, const double *df2,
-                            const int *mtab, double *bes, double *atab, double *nodes);
+hipError_t launch_species_k(hipStream_t st, int nspec, const TabSet &T, const int *mtab);
 hipError_t launch_sweep(hipStream_t st, int nch, int W, int RC, const ProbDev *prob, int nom,
                         const double2 *om, const int *active, double2 *chiA, double2 *lowA,
                         int npar1, const int *pidx = nullptr, unsigned long long *work = nullptr);
@@ -54,12 +51,8 @@ hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob,
 hipError_t launch_nhds(hipStream_t st, const ProbDev *prob, int nspec, int nom, const double2 *om,
                        const int *active, double2 *chiA, double2 *lowA, const int *pidx = nullptr);
 int nhds_tables(double z, int bm_nmax, double bessel_zero, std::vector<double2> &tab);
-hipError_t launch_lsum(hipStream_t st, int nperp, int nmax, double dpp, const double *pperp,
-                       const double *fitc, const double *atab, double *lsum);
 hipError_t launch_fill_i32(hipStream_t st, int *p, int n, int v);
-hipError_t launch_split_tables(hipStream_t st, int npar, int nmax, double kpar, double q, double m,
-                               const double *ppar, const double *nodes, double *crec,
-                               double *rsum, double *gcum);
+hipError_t launch_split_tables(hipStream_t st, int nspec, const TabSet &T);
 hipError_t launch_series_tables(hipStream_t st, int npar, int nmax, double kpar, double q, double m,
                                 const double *ppar, const double *nodes, double *ser, double *serD);
 hipError_t launch_rel_bessel(hipStream_t st, int npts, int nmax, double zfac, const double *grel,
@@ -196,11 +189,13 @@ struct alpsg_ctx {
   DevBuf<int> mtab;
   std::vector<double> int_ee_h;
   // per-k device data
-  DevBuf<double> bes[ALPSG_MAXSPEC], atab[ALPSG_MAXSPEC], nodes[ALPSG_MAXSPEC];
+  DevBuf<double> atab[ALPSG_MAXSPEC], nodes[ALPSG_MAXSPEC];
   DevBuf<double> crec[ALPSG_MAXSPEC], rsum[ALPSG_MAXSPEC];  // split-form sweep tables
   DevBuf<double> gcum[ALPSG_MAXSPEC];  // cumulative G/m sums (partial-range split rows)
   DevBuf<double> ser[ALPSG_MAXSPEC], serD[ALPSG_MAXSPEC];  // far-row series tables
   bool series_on = true;    // far rows of the node sweep take their series
+  TabSet tabset;               // the current k's table jobs
+  bool split_pending = false;  // the current k's split-form tables are not built yet
   bool ser_pending = false;  // the current k's series tables are not built yet
   bool ser_built = false;    // they are (the buffers hold this k's tables)
   DevBuf<double> lsum[ALPSG_MAXSPEC];  // Landau sums of single-Maxwellian species
@@ -296,7 +291,6 @@ struct alpsg_ctx {
     mval_d.release();
     mhit_d.release();
     for (int s = 0; s < ALPSG_MAXSPEC; ++s) {
-      bes[s].release();
       atab[s].release();
       nodes[s].release();
       crec[s].release();
@@ -435,6 +429,15 @@ bool shape_is_valid(const int *t) {
   return a && b && t[2] >= 1 && t[2] <= 64 && t[4] >= 1 && t[4] <= 16 && t[1] * t[2] <= 128;
 }
 
+// The split-form tables of the current k (13 us of launches a species, which a
+// scan's steps do not read), before a launch of the one-lane sweep.
+int ensure_split(alpsg_ctx *h, int nch_a) {
+  if (!h->split_pending || nch_a != 1) return ALPSG_OK;
+  HIPCHK(launch_split_tables(h->st, h->nspec, h->tabset));
+  h->split_pending = false;
+  return ALPSG_OK;
+}
+
 // The device buffers of one disp chain (det, the partial-chi slots, and for
 // small batches the zero problem indices of the request sweep).
 struct DispBufs {
@@ -455,6 +458,8 @@ int disp_chain(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_dev
   // omega's row pairs over REQ_TW wavefronts (problem index 0 for every omega).
   // The n_s-row partial layout is the same, so the rest of the chain is unchanged.
   const bool req = !want_low && active_dev == nullptr && n <= REQ_MAX_N;
+  if (!req)
+    if (const int rc = ensure_split(h, sh.nch_a)) return rc;
   if (req) {
     HIPCHK(launch_sweep_req(h->st, REQ_NCH, REQ_W, REQ_TW / REQ_W, REQ_K, h->prob_d.p, n, om_dev,
                             B.chiA, B.zidx, true));
@@ -705,7 +710,8 @@ namespace {
 int autotune(alpsg_ctx *h, int n, const double2 *om_host, int *shape_out) {
   if (!h->have_k) return fail(ALPSG_E_STATE, "alpsg_set_k has not been called");
   if (n < 1) return fail(ALPSG_E_ARG, "n must be >= 1");
-  if (const int rc = ensure_series(h, n)) return rc;  // the variants are timed as they will run
+  if (const int rc = ensure_split(h, 1)) return rc;  // the variants are timed as they will run
+  if (const int rc = ensure_series(h, n)) return rc;
   std::vector<double2> om(n);
   if (om_host) {
     for (int i = 0; i < n; ++i) om[i] = om_host[i];
@@ -981,6 +987,8 @@ int osc_graph_batch(alpsg_ctx *h, const alpsg_root_params *rp, int n, cplx *om, 
   const int ns = h->nspec;
   LaunchShape sh = shape_for(h, n);
   const bool req = n <= REQ_MAX_N;
+  if (!req)
+    if (const int rc = ensure_split(h, sh.nch_a)) return rc;
   const int TW = req ? REQ_TW / REQ_W : sh.w_a * sh.rc_a;  // partial slots of the sweep
   const int shp[5] = {sh.nch_a, sh.w_a, sh.rc_a, sh.nch_b, sh.rb};
   HIPCHK(h->om_d.ensure(std::max(n, REQ_MAX_N)));
@@ -2188,6 +2196,9 @@ int alpsg_set_k(alpsg_handle h, double kperp, double kpar, const int *nmax_in, i
     }
   }
   int nmaxR = 0;
+  TabSet &T = h->tabset;
+  std::memset(&T, 0, sizeof(T));
+  for (int s = 0; s < ALPSG_DMAXSPEC; ++s) T.j[s].nmax = -1;
   for (int s = 0; s < nspec; ++s) {
     SpecDev &S = h->prob.sp[s];
     const int nm = nmax[s];
@@ -2209,14 +2220,22 @@ int alpsg_set_k(alpsg_handle h, double kperp, double kpar, const int *nmax_in, i
       S.nmax = -1;
       continue;
     }
-    HIPCHK(h->bes[s].ensure((size_t)(nm + 3) * (nperp + 1)));
     HIPCHK(h->atab[s].ensure((size_t)(nm + 1) * (nperp + 1) * ATAB_STRIDE));
     HIPCHK(h->nodes[s].ensure((size_t)(nm + 1) * (npar - 1) * NODE_STRIDE));
-    HIPCHK(launch_species_k(h->st, nperp, npar, nm, kperp, kpar, h->qs[s], h->ms[s],
-                            h->pperp.p + (size_t)s * (nperp + 1), h->ppar.p + (size_t)s * (npar + 1),
-                            h->df1.p + (size_t)s * (nperp + 1) * (npar + 1),
-                            h->df2.p + (size_t)s * (nperp + 1) * (npar + 1), h->mtab.p, h->bes[s].p,
-                            h->atab[s].p, h->nodes[s].p));
+    TabJob &J = T.j[s];
+    J.pperp = h->pperp.p + (size_t)s * (nperp + 1);
+    J.ppar = h->ppar.p + (size_t)s * (npar + 1);
+    J.df1 = h->df1.p + (size_t)s * (nperp + 1) * (npar + 1);
+    J.df2 = h->df2.p + (size_t)s * (nperp + 1) * (npar + 1);
+    J.atab = h->atab[s].p;
+    J.nodes = h->nodes[s].p;
+    J.kperp = kperp;
+    J.kpar = kpar;
+    J.q = h->qs[s];
+    J.m = h->ms[s];
+    J.nperp = nperp;
+    J.npar = npar;
+    J.nmax = nm;
     S.nmax = nm;
     S.z = h->kperp_norm ? kperp / h->qs[s] : 1.0 / h->qs[s];
     S.atab = h->atab[s].p;
@@ -2226,8 +2245,9 @@ int alpsg_set_k(alpsg_handle h, double kperp, double kpar, const int *nmax_in, i
     S.lsum = nullptr;
     if (!h->relsp[s] && S.acmethod == 1 && S.fit_uniform && S.nfits == 1) {
       HIPCHK(h->lsum[s].ensure((size_t)(nm + 1) * 6));
-      HIPCHK(launch_lsum(h->st, nperp, nm, S.dpperp, h->pperp.p + (size_t)s * (nperp + 1), S.fitc,
-                         h->atab[s].p, h->lsum[s].p));
+      T.fitc[s] = S.fitc;
+      T.dpperp[s] = S.dpperp;
+      T.lsum[s] = h->lsum[s].p;
       S.lsum = h->lsum[s].p;
     }
     if (!h->relsp[s]) {
@@ -2236,9 +2256,9 @@ int alpsg_set_k(alpsg_handle h, double kperp, double kpar, const int *nmax_in, i
       HIPCHK(h->gcum[s].ensure((size_t)(nm + 1) * npar * GCUM_STRIDE));
       HIPCHK(h->ser[s].ensure((size_t)(nm + 1) * 2 * SER_Q * SER_STRIDE));
       HIPCHK(h->serD[s].ensure((size_t)(nm + 1) * 2));
-      HIPCHK(launch_split_tables(h->st, npar, nm, kpar, h->qs[s], h->ms[s],
-                                 h->ppar.p + (size_t)s * (npar + 1), h->nodes[s].p, h->crec[s].p,
-                                 h->rsum[s].p, h->gcum[s].p));
+      T.crec[s] = h->crec[s].p;
+      T.rsum[s] = h->rsum[s].p;
+      T.gcum[s] = h->gcum[s].p;
       S.crec = h->crec[s].p;
       S.rsum = h->rsum[s].p;
       S.gcum = h->gcum[s].p;
@@ -2260,6 +2280,8 @@ int alpsg_set_k(alpsg_handle h, double kperp, double kpar, const int *nmax_in, i
       nmaxR = std::max(nmaxR, nm);
     }
   }
+  HIPCHK(launch_species_k(h->st, nspec, T, h->mtab.p));
+  h->split_pending = true;  // built by the first launch that reads them (ensure_split)
   h->prob.kperp = kperp;
   h->prob.kpar = kpar;
   h->prob.nmaxR = nmaxR;
@@ -2394,6 +2416,7 @@ int alpsg_sweep_work(alpsg_handle h, int n, const double *om, double *work3) {
   for (int k = 0; k < 3; ++k) work3[k] = 0.0;
   if (n == 0) return ALPSG_OK;
   const LaunchShape sh = shape_for(h, n);
+  if (const int rc = ensure_split(h, sh.nch_a)) return rc;
   if (const int rc = ensure_series(h, n)) return rc;
   HIPCHK(h->om_d.ensure(n));
   HIPCHK(h->chiA_d.ensure((size_t)n * sh.w_a * sh.rc_a * h->nspec * 6));

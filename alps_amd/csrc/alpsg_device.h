@@ -96,6 +96,16 @@ struct TabJob {
   int nperp, npar, nmax, ntry;
 };
 
+// The species of one set_k: their table jobs (nmax < 0: no tables, bmax and bes
+// unused) and the further tables of the handle.
+struct TabSet {
+  TabJob j[ALPSG_DMAXSPEC];
+  const double *fitc[ALPSG_DMAXSPEC];  // lsum's fit rows
+  double dpperp[ALPSG_DMAXSPEC];
+  double *lsum[ALPSG_DMAXSPEC];                        // NULL: none
+  double *crec[ALPSG_DMAXSPEC], *rsum[ALPSG_DMAXSPEC], *gcum[ALPSG_DMAXSPEC];  // NULL: none
+};
+
 struct ProbDev {
   int nspec, kperp_norm, P, NRI;
   double kperp, kpar, vA, Tlim;

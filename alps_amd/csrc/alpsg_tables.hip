@@ -3,8 +3,8 @@
 //   k_derivative   df0 from f0 (derivative_f0, ALPS_fns.f90:103-115)
 //   k_int_ee       omega-independent ee term (int_ee, ALPS_fns.f90:1457-1555)
 //   k_bessel_max   max_iperp |J_n| for n = 1..ntry (determine_nmax, ALPS_fns.f90:4017-4035)
-//   k_bessel       J_n table, n = -1..nmax+1 (determine_bessel_array, ALPS_fns.f90:4214-4255)
-//   k_atab         J^2, pperp^2 J'^2, pperp J J' per (n, iperp) (int_T, ALPS_fns.f90:1639-1707)
+//   k_atab         J_n (determine_bessel_array, ALPS_fns.f90:4214-4255) and
+//                  J^2, pperp^2 J'^2, pperp J J' per (n, iperp) (int_T, ALPS_fns.f90:1639-1707)
 //   k_moments      pperp-reduced node tables G_a(n,ipar), H_a(n,ipar)
 //
 // The pperp moments rest on the factorisation of resU*int_T
@@ -220,27 +220,12 @@ __device__ __forceinline__ void bessel_entry(int ip, int n, int nperp, int nmax,
   bes[(size_t)(n + 1) * (nperp + 1) + ip] = v;
 }
 
-__global__ void k_bessel(int nperp, int nmax, double kperp, double q,
-                         const double *__restrict__ pperp, const int *__restrict__ mtab,
-                         double *__restrict__ bes) {
-  bessel_entry(blockIdx.x * blockDim.x + threadIdx.x, (int)blockIdx.y - 1, nperp, nmax, kperp, q,
-               pperp, mtab, bes);
-}
-
 // a-types per (n >= 0, iperp): J^2, pperp^2 J'^2, pperp J J', J.
 // J'_n = (J_{n-1} - J_{n+1})/2 for n >= 1, -J_1 for n = 0 (int_T, ALPS_fns.f90:1647-1656).
 // The negative harmonics use the same values: J_{-n}^2 = J_n^2 and
 // J_{-n} J'_{-n} = J_n J'_n exactly in floating point.
-__device__ __forceinline__ void atab_entry(int ip, int n, int nperp, int nmax,
-                                           const double *__restrict__ pperp,
-                                           const double *__restrict__ bes,
-                                           double *__restrict__ atab) {
-  if (ip > nperp || n > nmax) return;
-  const int W = nperp + 1;
-  double J = bes[(size_t)(n + 1) * W + ip];
-  double Jp = (n >= 1) ? 0.5 * (bes[(size_t)n * W + ip] - bes[(size_t)(n + 2) * W + ip])
-                       : -bes[(size_t)2 * W + ip];
-  double p = pperp[ip];
+__device__ __forceinline__ void atab_put(int n, int ip, int W, double J, double Jp, double p,
+                                         double *__restrict__ atab) {
   double *o = atab + ((size_t)n * W + ip) * ATAB_STRIDE;
   o[0] = J * J;
   o[1] = (p * p) * Jp * Jp;
@@ -248,104 +233,85 @@ __device__ __forceinline__ void atab_entry(int ip, int n, int nperp, int nmax,
   o[3] = J;
 }
 
-__global__ void k_atab(int nperp, int nmax, const double *__restrict__ pperp,
-                       const double *__restrict__ bes, double *__restrict__ atab) {
-  atab_entry(blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, nperp, nmax, pperp, bes, atab);
+__device__ __forceinline__ void atab_entry(int ip, int n, int nperp, int nmax,
+                                           const double *__restrict__ pperp,
+                                           const double *__restrict__ bes,
+                                           double *__restrict__ atab) {
+  if (ip > nperp || n > nmax) return;
+  const int W = nperp + 1;
+  const double Jp = (n >= 1) ? 0.5 * (bes[(size_t)n * W + ip] - bes[(size_t)(n + 2) * W + ip])
+                             : -bes[(size_t)2 * W + ip];
+  atab_put(n, ip, W, bes[(size_t)(n + 1) * W + ip], Jp, pperp[ip], atab);
+}
+
+// The per-k tables of a handle, every species in one launch each (grid z): their
+// time is the latency of a few hundred wavefronts, not work, and species after
+// species they were most of what a step of a kpar scan spends outside its secant
+// rounds (two species of 50 x 100: 114 us of seven kernels each, now 17 us;
+// three of 128 x 256: 288 us, now 29 us).
+
+// J and the a-types of BT harmonics at 64 pperp points: wavefront w takes J of
+// harmonic n0 - 1 + w, the first BT of them an a-row each
+constexpr int BT = 6;
+__global__ __launch_bounds__((BT + 2) * 64) void k_atab(TabSet T, const int *__restrict__ mtab) {
+  __shared__ double Jl[BT + 2][64];
+  const TabJob &J = T.j[blockIdx.z];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int ip = blockIdx.x * 64 + l, n0 = blockIdx.y * BT, W = J.nperp + 1;
+  if (n0 > J.nmax || (int)blockIdx.x * 64 > J.nperp) return;
+  const double p = J.pperp[min(ip, J.nperp)];
+  const int n = n0 - 1 + w;
+  if (n >= 0 && n <= J.nmax + 1) Jl[w][l] = dev_bessj(n, J.kperp * p / J.q, mtab);
+  __syncthreads();
+  const int an = n0 + w;
+  if (w >= BT || an > J.nmax || ip > J.nperp) return;
+  const double Jp = an >= 1 ? 0.5 * (Jl[w][l] - Jl[w + 2][l]) : -Jl[w + 2][l];
+  atab_put(an, ip, W, Jl[w + 1][l], Jp, p, J.atab);
 }
 
 // Landau sums of a single-Maxwellian species (the omega-independent part of
 // landau_integrate, ALPS_fns.f90:1382-1444, when eval_fit = c0(iperp) E(p)):
 // with dfpar = c0 (E(p+d) - E(p-d))/2d and dfperp = beta E(p), the sum over
 // iperp of h a K is qk [km A sum(h a pperp c0) + (om - km p) E(p) sum(h a beta)],
-// A = (E(p+d) - E(p-d))/2d.  One thread per (n, sum), iperp in order.
-__global__ void k_lsum(int nperp, int nmax, double dpp, const double *__restrict__ pperp,
-                       const double *__restrict__ fitc, const double *__restrict__ atab,
-                       double *__restrict__ lsum) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 6 * (nmax + 1)) return;
+// A = (E(p+d) - E(p-d))/2d.  One lane per (n, sum), iperp in order; the rows'
+// factors come from LDS and the a-values LU rows at a time, so that a row costs
+// its arithmetic and not a load's latency.
+constexpr int LU = 16;
+__device__ __forceinline__ void lsum_block(int b, const TabJob &J, double dpp,
+                                           const double *__restrict__ fitc,
+                                           double *__restrict__ lsum) {
+  __shared__ double v[2][64];
+  const int nperp = J.nperp, W = nperp + 1, l = threadIdx.x, nt = 6 * (J.nmax + 1);
+  const int t = min(b * 64 + l, nt - 1);
   const int n = t / 6, w = t % 6, k = w % 3;
-  const int W = nperp + 1;
+  const double *at = J.atab + (size_t)n * W * ATAB_STRIDE + k;
   auto c0 = [&](int ip) { return fitc[(size_t)ip * FIT_STRIDE]; };
   double acc = 0.0;
-  for (int ip = 0; ip <= nperp; ++ip) {
-    const double h = (ip == 0 || ip >= nperp - 1) ? 0.5 : 1.0;
-    const double a = atab[((size_t)n * W + ip) * ATAB_STRIDE + k];
-    double v;
-    if (w < 3) {
-      v = pperp[ip] * c0(ip);
-    } else if (ip == 0) {
-      v = (c0(1) - c0(0)) * (1.0 / dpp);
-    } else if (ip == nperp) {
-      v = (c0(nperp) - c0(nperp - 1)) * (1.0 / dpp);
-    } else {
-      v = (c0(ip + 1) - c0(ip - 1)) * (1.0 / (2.0 * dpp));
+  for (int r0 = 0; r0 <= nperp; r0 += 64) {
+    __syncthreads();
+    const int ip = min(r0 + l, nperp);
+    v[0][l] = J.pperp[ip] * c0(ip);
+    if (ip == 0)
+      v[1][l] = (c0(1) - c0(0)) * (1.0 / dpp);
+    else if (ip == nperp)
+      v[1][l] = (c0(nperp) - c0(nperp - 1)) * (1.0 / dpp);
+    else
+      v[1][l] = (c0(ip + 1) - c0(ip - 1)) * (1.0 / (2.0 * dpp));
+    __syncthreads();
+    for (int u0 = 0; u0 < 64 && r0 + u0 <= nperp; u0 += LU) {
+      double a[LU];
+#pragma unroll
+      for (int u = 0; u < LU; ++u) a[u] = at[(size_t)min(r0 + u0 + u, nperp) * ATAB_STRIDE];
+#pragma unroll
+      for (int u = 0; u < LU; ++u) {
+        const int i = r0 + u0 + u;
+        if (i > nperp) break;
+        const double h = (i == 0 || i >= nperp - 1) ? 0.5 : 1.0;
+        acc += (h * a[u]) * v[w < 3 ? 0 : 1][u0 + u];
+      }
     }
-    acc += (h * a) * v;
   }
-  lsum[t] = acc;
-}
-
-hipError_t launch_lsum(hipStream_t st, int nperp, int nmax, double dpp, const double *pperp,
-                       const double *fitc, const double *atab, double *lsum) {
-  const int n = 6 * (nmax + 1);
-  hipLaunchKernelGGL(k_lsum, dim3((n + 63) / 64), dim3(64), 0, st, nperp, nmax, dpp, pperp, fitc,
-                     atab, lsum);
-  return hipGetLastError();
-}
-
-// Node tables: one thread per (n, ipar), summing over iperp.  The a-values of a
-// given n are shared by the whole block (staged in LDS); df1/df2 rows are read
-// coalesced along ipar.
-__device__ __forceinline__ void moments_block(int bx, int n, int nperp, int npar, double kpar,
-                                              double m, const double *__restrict__ pperp,
-                                              const double *__restrict__ ppar,
-                                              const double *__restrict__ df1,
-                                              const double *__restrict__ df2,
-                                              const double *__restrict__ atab,
-                                              double *__restrict__ nodes, double *lds_a) {
-  int ipar = 1 + bx * blockDim.x + threadIdx.x;
-  const int W = nperp + 1;
-  for (int t = threadIdx.x; t < (nperp - 1); t += blockDim.x) {
-    const double *a = atab + ((size_t)n * W + (t + 1)) * ATAB_STRIDE;
-    double wperp = (t + 1 == nperp - 1) ? 1.0 : 2.0;
-    lds_a[3 * t + 0] = wperp * a[0];
-    lds_a[3 * t + 1] = wperp * a[1];
-    lds_a[3 * t + 2] = wperp * a[2];
-  }
-  __syncthreads();
-  if (ipar > npar - 1) return;
-  double pa = ppar[ipar];
-  double kom = kpar / m;
-  double g1 = 0, h1 = 0, g2 = 0, h2 = 0, g3 = 0, h3 = 0;
-  for (int iperp = 1; iperp <= nperp - 1; ++iperp) {
-    size_t o = (size_t)iperp * (npar + 1) + ipar;
-    double d1 = df1[o], d2 = df2[o];
-    double A = kom * (pperp[iperp] * d2 - pa * d1);
-    double a1 = lds_a[3 * (iperp - 1) + 0], a2 = lds_a[3 * (iperp - 1) + 1],
-           a3 = lds_a[3 * (iperp - 1) + 2];
-    g1 += a1 * d1;
-    h1 += a1 * A;
-    g2 += a2 * d1;
-    h2 += a2 * A;
-    g3 += a3 * d1;
-    h3 += a3 * A;
-  }
-  double *o = nodes + ((size_t)n * (npar - 1) + (ipar - 1)) * NODE_STRIDE;
-  o[0] = g1;
-  o[1] = h1;
-  o[2] = g2;
-  o[3] = h2;
-  o[4] = g3;
-  o[5] = h3;
-}
-
-__global__ void k_moments(int nperp, int npar, int nmax, double kpar, double m,
-                          const double *__restrict__ pperp, const double *__restrict__ ppar,
-                          const double *__restrict__ df1, const double *__restrict__ df2,
-                          const double *__restrict__ atab, double *__restrict__ nodes) {
-  extern __shared__ double lds_a[];  // (nperp-1) * 3
-  moments_block(blockIdx.x, blockIdx.y, nperp, npar, kpar, m, pperp, ppar, df1, df2, atab, nodes,
-                lds_a);
+  if (b * 64 + l < nt) lsum[t] = acc;
 }
 
 // Split-form records of the one-lane-per-omega sweep.  With den = m w - kpar p
@@ -353,12 +319,15 @@ __global__ void k_moments(int nperp, int npar, int nmax, double kpar, double m,
 //   U_a / den = G_a / m + C_a / den,  C_a = G_a (kpar p +- n q) / m + H_a,
 // where C_a is real and omega-independent.  Record (n, ipar):
 //   [0] kpar p, [1..6] C1, p C1, p^2 C1, C2, C3, p C3 for +n, [7..12] for -n.
-__global__ void k_crec(int npar, int nmax, double kpar, double q, double m,
-                       const double *__restrict__ ppar, const double *__restrict__ nodes,
-                       double *__restrict__ crec) {
+__global__ void k_crec(TabSet T) {
+  const TabJob &J = T.j[blockIdx.z];
+  const int npar = J.npar, nmax = J.nmax;
+  const double kpar = J.kpar, q = J.q, m = J.m;
+  const double *__restrict__ ppar = J.ppar, *__restrict__ nodes = J.nodes;
+  double *__restrict__ crec = T.crec[blockIdx.z];
   const int ipar = 1 + blockIdx.x * blockDim.x + threadIdx.x;
   const int n = blockIdx.y;
-  if (ipar > npar - 1 || n > nmax) return;
+  if (ipar > npar - 1 || n > nmax || crec == nullptr) return;
   const double *r = nodes + ((size_t)n * (npar - 1) + (ipar - 1)) * NODE_STRIDE;
   const double p = ppar[ipar], p2 = p * p;
   const double kp = kpar * p, nq = (1.0 * n) * q;
@@ -380,11 +349,14 @@ __global__ void k_crec(int npar, int nmax, double kpar, double q, double m,
 // rsum[n] = sum over the interior nodes ipar = 2..npar-2 of
 // {G1, p G1, p^2 G1, G2, G3, p G3} / m: one wavefront per harmonic, lanes
 // strided over the nodes, then a fixed-order butterfly over the lanes
-__global__ __launch_bounds__(64) void k_rsum(int npar, int nmax, double m,
-                                             const double *__restrict__ ppar,
-                                             const double *__restrict__ nodes,
-                                             double *__restrict__ rsum) {
+__global__ __launch_bounds__(64) void k_rsum(TabSet T) {
+  const TabJob &J = T.j[blockIdx.y];
+  const int npar = J.npar, nmax = J.nmax;
+  const double m = J.m;
+  const double *__restrict__ ppar = J.ppar, *__restrict__ nodes = J.nodes;
+  double *__restrict__ rsum = T.rsum[blockIdx.y];
   const int n = blockIdx.x, lane = threadIdx.x;
+  if (n > nmax || rsum == nullptr) return;
   double a[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   for (int ipar = 2 + lane; ipar <= npar - 2; ipar += 64) {
     const double *r = nodes + ((size_t)n * (npar - 1) + (ipar - 1)) * NODE_STRIDE;
@@ -482,11 +454,14 @@ __global__ __launch_bounds__(256) void k_series(int npar, int nmax, double kpar,
 // gcum[n][i] = sum over ipar = 1..i of {G1, p G1, p^2 G1, G2, G3, p G3} / m,
 // gcum[n][0] = 0: one wavefront per harmonic, an inclusive lane scan per
 // chunk of 64 nodes plus the running carry
-__global__ __launch_bounds__(64) void k_gcum(int npar, int nmax, double m,
-                                             const double *__restrict__ ppar,
-                                             const double *__restrict__ nodes,
-                                             double *__restrict__ gcum) {
+__global__ __launch_bounds__(64) void k_gcum(TabSet T) {
+  const TabJob &J = T.j[blockIdx.y];
+  const int npar = J.npar, nmax = J.nmax;
+  const double m = J.m;
+  const double *__restrict__ ppar = J.ppar, *__restrict__ nodes = J.nodes;
+  double *__restrict__ gcum = T.gcum[blockIdx.y];
   const int n = blockIdx.x, lane = threadIdx.x;
+  if (n > nmax || gcum == nullptr) return;
   double *g = gcum + (size_t)n * npar * GCUM_STRIDE;
   if (lane < GCUM_STRIDE) g[lane] = 0.0;
   double carry[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -521,13 +496,17 @@ __global__ __launch_bounds__(64) void k_gcum(int npar, int nmax, double m,
   }
 }
 
-hipError_t launch_split_tables(hipStream_t st, int npar, int nmax, double kpar, double q, double m,
-                               const double *ppar, const double *nodes, double *crec,
-                               double *rsum, double *gcum) {
-  hipLaunchKernelGGL(k_crec, dim3((npar - 1 + 63) / 64, nmax + 1), dim3(64), 0, st, npar, nmax,
-                     kpar, q, m, ppar, nodes, crec);
-  hipLaunchKernelGGL(k_rsum, dim3(nmax + 1), dim3(64), 0, st, npar, nmax, m, ppar, nodes, rsum);
-  hipLaunchKernelGGL(k_gcum, dim3(nmax + 1), dim3(64), 0, st, npar, nmax, m, ppar, nodes, gcum);
+hipError_t launch_split_tables(hipStream_t st, int nspec, const TabSet &T) {
+  int npar = 0, nmax = -1;
+  for (int s = 0; s < nspec; ++s)
+    if (T.crec[s] != nullptr) {
+      npar = max(npar, T.j[s].npar);
+      nmax = max(nmax, T.j[s].nmax);
+    }
+  if (nmax < 0) return hipSuccess;
+  hipLaunchKernelGGL(k_crec, dim3((npar - 1 + 63) / 64, nmax + 1, nspec), dim3(64), 0, st, T);
+  hipLaunchKernelGGL(k_rsum, dim3(nmax + 1, nspec), dim3(64), 0, st, T);
+  hipLaunchKernelGGL(k_gcum, dim3(nmax + 1, nspec), dim3(64), 0, st, T);
   return hipGetLastError();
 }
 
@@ -586,129 +565,18 @@ __global__ void k_atab_jobs(const TabJob *__restrict__ jobs, const int *__restri
   atab_entry(bx * 64 + threadIdx.x, by, J.nperp, J.nmax, J.pperp, J.bes, J.atab);
 }
 
-// moments_block for MB consecutive harmonics n0 .. n0+MB-1 (those above nmax
-// are computed on n = nmax and not stored): every df0 load serves MB
-// harmonics.  The weighted a-values of the block's harmonics and the pperp
-// values are staged in LDS MCH rows at a time (one row per lane, its loads all
-// in flight together), so the row loop reads them as LDS broadcasts instead of
-// a chain of dependent scalar loads per row.  Sums run over iperp in order, as
-// in moments_block.
-constexpr int MB = 8;
-constexpr int MCH = 64;
-constexpr int MR = 4;
-typedef const __attribute__((address_space(1))) double *gdptr_t;
-
-__device__ __forceinline__ void moments_row(double (&g)[MB][3], double (&h)[MB][3],
-                                            const double *la_row, double pe, double d1, double d2,
-                                            double kom, double pa) {
-  const double A = kom * (pe * d2 - pa * d1);
-#pragma unroll
-  for (int u = 0; u < MB; ++u) {
-    const double a1 = la_row[3 * u + 0], a2 = la_row[3 * u + 1], a3 = la_row[3 * u + 2];
-    g[u][0] += a1 * d1;
-    h[u][0] += a1 * A;
-    g[u][1] += a2 * d1;
-    h[u][1] += a2 * A;
-    g[u][2] += a3 * d1;
-    h[u][2] += a3 * A;
-  }
-}
-
-__device__ __forceinline__ void moments_block_mb(int bx, int n0, int nperp, int npar, int nmax,
-                                                 double kpar, double m,
-                                                 const double *__restrict__ pperp,
-                                                 const double *__restrict__ ppar,
-                                                 const double *__restrict__ df1,
-                                                 const double *__restrict__ df2,
-                                                 const double *__restrict__ atab,
-                                                 double *__restrict__ nodes) {
-  __shared__ double la[MCH][MB * 3];
-  __shared__ double lpe[MCH];
-  const int ipar = 1 + bx * 64 + threadIdx.x;
-  const int ip = ipar <= npar - 1 ? ipar : npar - 1;
-  const int W = nperp + 1;
-  const double pa = ppar[ip];
-  const double kom = kpar / m;
-  // global (not flat) loads: their waits do not hold the LDS reads
-  const gdptr_t f1 = (gdptr_t)df1, f2 = (gdptr_t)df2;
-  double g[MB][3], h[MB][3];
-#pragma unroll
-  for (int u = 0; u < MB; ++u)
-#pragma unroll
-    for (int t = 0; t < 3; ++t) g[u][t] = h[u][t] = 0.0;
-  for (int c0 = 1; c0 <= nperp - 1; c0 += MCH) {
-    const int cn = min(MCH, nperp - c0);  // rows c0 .. c0 + cn - 1 <= nperp - 1
-    __syncthreads();                       // the previous chunk is consumed
-    if ((int)threadIdx.x < cn) {
-      const int iperp = c0 + threadIdx.x;
-      const double wperp = (iperp == nperp - 1) ? 1.0 : 2.0;
-      double v[MB * 3];
-#pragma unroll
-      for (int u = 0; u < MB; ++u) {
-        const double *a = atab + ((size_t)min(n0 + u, nmax) * W + iperp) * ATAB_STRIDE;
-        v[3 * u + 0] = a[0];
-        v[3 * u + 1] = a[1];
-        v[3 * u + 2] = a[2];
-      }
-#pragma unroll
-      for (int k = 0; k < MB * 3; ++k) la[threadIdx.x][k] = wperp * v[k];
-      lpe[threadIdx.x] = pperp[iperp];
-    }
-    __syncthreads();
-    // rows in groups of MR, the group's df loads issued before its sums, then
-    // the remaining rows one by one
-    int t0 = 0;
-    for (; t0 + MR <= cn; t0 += MR) {
-      double d1[MR], d2[MR];
-#pragma unroll
-      for (int r = 0; r < MR; ++r) {
-        const size_t o = (size_t)(c0 + t0 + r) * (npar + 1) + ip;
-        d1[r] = f1[o];
-        d2[r] = f2[o];
-      }
-#pragma unroll
-      for (int r = 0; r < MR; ++r) moments_row(g, h, la[t0 + r], lpe[t0 + r], d1[r], d2[r], kom, pa);
-    }
-    for (; t0 < cn; ++t0) {
-      const size_t o = (size_t)(c0 + t0) * (npar + 1) + ip;
-      moments_row(g, h, la[t0], lpe[t0], f1[o], f2[o], kom, pa);
-    }
-  }
-  if (ipar > npar - 1) return;
-#pragma unroll
-  for (int u = 0; u < MB; ++u) {
-    const int n = n0 + u;
-    if (n > nmax) break;
-    double *o = nodes + ((size_t)n * (npar - 1) + (ipar - 1)) * NODE_STRIDE;
-    o[0] = g[u][0];
-    o[1] = h[u][0];
-    o[2] = g[u][1];
-    o[3] = h[u][1];
-    o[4] = g[u][2];
-    o[5] = h[u][2];
-  }
-}
-
-__global__ __launch_bounds__(64) void k_moments_jobs(const TabJob *__restrict__ jobs,
-                                                     const int *__restrict__ start, int njobs) {
-  const int j = job_of(start, njobs, blockIdx.x);
-  const TabJob &J = jobs[j];
-  const int b = blockIdx.x - start[j];
-  const int tiles = (J.npar - 1 + 63) / 64;
-  const int bx = b % tiles, by = b / tiles;
-  moments_block_mb(bx, by * MB, J.nperp, J.npar, J.nmax, J.kpar, J.m, J.pperp, J.ppar, J.df1,
-                   J.df2, J.atab, J.nodes);
-}
-
-// The same node tables on the matrix cores.  For one species the node sums
+// The node tables on the matrix cores.  For one species the node sums
 // are a real GEMM, nodes[(n, a)][(ipar, g/h)] = sum_iperp Aw[(n, a)][iperp]
 // B[iperp][(ipar, g/h)], with Aw = w_perp a(n, iperp) (a = J^2, pperp^2 J'^2,
 // pperp J J'), B(g) = df1 and B(h) = (kpar/m)(pperp df2 - ppar df1) per point,
 // M = 3 (nmax+1), N = 2 (npar-1), K = nperp-1.  One wavefront computes a
 // 16 x 16 MT tile with v_mfma_f64_16x16x4f64 (lane l holds A[l%16][l/16] and
 // B[l/16][l%16], and D[l/16 + 4q][l%16] in element q), stepping K by 4;
-// elements outside M, N or K enter as zeros.  The per-point B values are
-// rounded as in moments_block; only the order of the sums over iperp differs.
+// elements outside M, N or K enter as zeros.  The operands of MK steps are loaded
+// before the first of them is used: a step's products take 16 cycles each and its
+// loads' latency some hundred (the tables of 512 served requests on four
+// grids 1230 us one step at a time, 820 us so).
+constexpr int MK = 4;
 constexpr int MT = 4;  // 16-column tiles per wavefront (one A operand feeds MT products)
 
 __device__ __forceinline__ void moments_mfma_tile(int tile_c, int tile_r, int nperp, int npar,
@@ -742,20 +610,33 @@ __device__ __forceinline__ void moments_mfma_tile(int tile_c, int tile_r, int np
   double4v acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = double4v{0.0, 0.0, 0.0, 0.0};
-  for (int k0 = 1; k0 <= nperp - 1; k0 += 4) {
-    const int iperp = k0 + kk;
-    const bool kv = iperp <= nperp - 1;
-    const int ik = kv ? iperp : 1;
-    const double wperp = (ik == nperp - 1) ? 1.0 : 2.0;
-    const double av = (rv && kv) ? wperp * atab[((size_t)an * W + ik) * ATAB_STRIDE + aa] : 0.0;
-    const double pe = pperp[ik];
+  const double *ar = atab + (size_t)an * W * ATAB_STRIDE + aa;
+  for (int k0 = 1; k0 <= nperp - 1; k0 += 4 * MK) {
+    double av[MK], pe[MK], d1[MK][MT], d2[MK][MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const size_t o = (size_t)ik * (npar + 1) + ipc[t];
-      const double d1 = df1[o], d2 = df2[o];
-      const double bg = ghc[t] ? kom * (pe * d2 - pac[t] * d1) : d1;
-      const double bv = (cv[t] && kv) ? bg : 0.0;
-      acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[t], 0, 0, 0);
+    for (int u = 0; u < MK; ++u) {
+      const int ik = min(k0 + 4 * u + kk, nperp - 1);
+      av[u] = ar[(size_t)ik * ATAB_STRIDE];
+      pe[u] = pperp[ik];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const size_t o = (size_t)ik * (npar + 1) + ipc[t];
+        d1[u][t] = df1[o];
+        d2[u][t] = df2[o];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < MK; ++u) {
+      if (k0 + 4 * u > nperp - 1) break;
+      const int ik = k0 + 4 * u + kk;
+      const bool kv = ik <= nperp - 1;
+      const double a = (rv && kv) ? ((ik == nperp - 1) ? 1.0 : 2.0) * av[u] : 0.0;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const double bg = ghc[t] ? kom * (pe[u] * d2[u][t] - pac[t] * d1[u][t]) : d1[u][t];
+        const double bv = (cv[t] && kv) ? bg : 0.0;
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bv, acc[t], 0, 0, 0);
+      }
     }
   }
 #pragma unroll
@@ -773,15 +654,20 @@ __device__ __forceinline__ void moments_mfma_tile(int tile_c, int tile_r, int np
   }
 }
 
-__global__ __launch_bounds__(64) void k_moments_mfma(int nperp, int npar, int nmax, double kpar,
-                                                     double m, const double *__restrict__ pperp,
-                                                     const double *__restrict__ ppar,
-                                                     const double *__restrict__ df1,
-                                                     const double *__restrict__ df2,
-                                                     const double *__restrict__ atab,
-                                                     double *__restrict__ nodes) {
-  moments_mfma_tile(blockIdx.x, blockIdx.y, nperp, npar, nmax, kpar, m, pperp, ppar, df1, df2,
-                    atab, nodes);
+__host__ __device__ inline int moments_tc(const TabJob &J) { return (2 * (J.npar - 1) + 16 * MT - 1) / (16 * MT); }
+__host__ __device__ inline int moments_tr(const TabJob &J) { return (3 * (J.nmax + 1) + 15) / 16; }
+
+// both tables that need the a-types: the node tables' tiles, then lsum's blocks
+__global__ __launch_bounds__(64) void k_moments(TabSet T) {
+  const int s = blockIdx.y;
+  const TabJob &J = T.j[s];
+  if (J.nmax < 0) return;
+  const int tc = moments_tc(J), nt = tc * moments_tr(J), b = blockIdx.x;
+  if (b < nt)
+    moments_mfma_tile(b % tc, b / tc, J.nperp, J.npar, J.nmax, J.kpar, J.m, J.pperp, J.ppar, J.df1,
+                      J.df2, J.atab, J.nodes);
+  else if (T.lsum[s] != nullptr && (b - nt) * 64 < 6 * (J.nmax + 1))
+    lsum_block(b - nt, J, T.dpperp[s], T.fitc[s], T.lsum[s]);
 }
 
 __global__ __launch_bounds__(64) void k_moments_mfma_jobs(const TabJob *__restrict__ jobs,
@@ -790,7 +676,7 @@ __global__ __launch_bounds__(64) void k_moments_mfma_jobs(const TabJob *__restri
   const int j = job_of(start, njobs, blockIdx.x);
   const TabJob &J = jobs[j];
   const int b = blockIdx.x - start[j];
-  const int tc = (2 * (J.npar - 1) + 16 * MT - 1) / (16 * MT);
+  const int tc = moments_tc(J);
   moments_mfma_tile(b % tc, b / tc, J.nperp, J.npar, J.nmax, J.kpar, J.m, J.pperp, J.ppar, J.df1,
                     J.df2, J.atab, J.nodes);
 }
@@ -857,18 +743,20 @@ hipError_t launch_rel_bessel(hipStream_t st, int npts, int nmax, double zfac, co
   return hipGetLastError();
 }
 
-hipError_t launch_species_k(hipStream_t st, int nperp, int npar, int nmax, double kperp,
-                            double kpar, double q, double m, const double *pperp,
-                            const double *ppar, const double *df1, const double *df2,
-                            const int *mtab, double *bes, double *atab, double *nodes) {
-  hipLaunchKernelGGL(k_bessel, dim3((nperp + 1 + 63) / 64, nmax + 3), dim3(64), 0, st, nperp,
-                     nmax, kperp, q, pperp, mtab, bes);
-  hipLaunchKernelGGL(k_atab, dim3((nperp + 1 + 63) / 64, nmax + 1), dim3(64), 0, st, nperp, nmax,
-                     pperp, bes, atab);
-  const int tc = (2 * (npar - 1) + 16 * MT - 1) / (16 * MT);
-  const int tr = (3 * (nmax + 1) + 15) / 16;
-  hipLaunchKernelGGL(k_moments_mfma, dim3(tc, tr), dim3(64), 0, st, nperp, npar, nmax, kpar, m,
-                     pperp, ppar, df1, df2, atab, nodes);
+hipError_t launch_species_k(hipStream_t st, int nspec, const TabSet &T, const int *mtab) {
+  int bt = 0, nmax = -1, nperp = 0;
+  for (int s = 0; s < nspec; ++s) {
+    const TabJob &J = T.j[s];
+    if (J.nmax < 0) continue;
+    nmax = max(nmax, J.nmax);
+    nperp = max(nperp, J.nperp);
+    bt = max(bt, moments_tc(J) * moments_tr(J) +
+                     (T.lsum[s] != nullptr ? (6 * (J.nmax + 1) + 63) / 64 : 0));
+  }
+  if (nmax < 0) return hipSuccess;
+  hipLaunchKernelGGL(k_atab, dim3((nperp + 1 + 63) / 64, nmax / BT + 1, nspec),
+                     dim3((BT + 2) * 64), 0, st, T, mtab);
+  hipLaunchKernelGGL(k_moments, dim3(bt, nspec), dim3(64), 0, st, T);
   return hipGetLastError();
 }
 
@@ -878,7 +766,7 @@ int jobs_blocks_bessel_max(const TabJob &J) { return J.ntry; }
 int jobs_blocks_bessel(const TabJob &J) { return ((J.nperp + 1 + 63) / 64) * (J.nmax + 3); }
 int jobs_blocks_atab(const TabJob &J) { return ((J.nperp + 1 + 63) / 64) * (J.nmax + 1); }
 int jobs_blocks_moments(const TabJob &J) {
-  return ((2 * (J.npar - 1) + 16 * MT - 1) / (16 * MT)) * ((3 * (J.nmax + 1) + 15) / 16);
+  return moments_tc(J) * moments_tr(J);
 }
 
 // start arrays: [njobs + 1] each, device copies; total = start[njobs]
