@@ -65,9 +65,9 @@ hipError_t launch_osc_round(hipStream_t st, int n, alpsg_osc::OscMachine *S, con
                             double2 *om, int *round_ctr, int *remaining);
 hipError_t launch_resonant_all(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec,
                                int nom, const double2 *om, double2 *chiB, int lgen);
-hipError_t launch_round(hipStream_t st, int nchr, int RB, int RC, const ProbDev *prob, int nspec,
+hipError_t launch_small(hipStream_t st, int nchr, int RB, int RC, const ProbDev *prob, int nspec,
                         int nom, double2 *om, double2 *chiA, double2 *chiB, double2 *det,
-                        const int *zidx, int lgen, alpsg_osc::OscMachine *S, int *ctl);
+                        const int *zidx, int lgen, int *done, alpsg_osc::OscMachine *S, int *ctl);
 hipError_t launch_assemble_osc(hipStream_t st, const ProbDev *prob, int nspec, int nom, int W, int RB,
                                double2 *om, const double2 *chiA, const double2 *chiB, double2 *det,
                                alpsg_osc::OscMachine *S, int *round_ctr, int *remaining);
@@ -202,15 +202,7 @@ struct alpsg_ctx {
   DevBuf<int> zidx;  // zeros: the problem index of every omega of a small batch
   DevBuf<unsigned long long> work_d;  // the sweep's work counts (alpsg_sweep_work)
   PinBuf om_pin, det_pin;  // staging of om and det for batches of at most PIN_MAX omegas
-  // captured disp chains of small batches (index n = 1..REQ_MAX_N), with the
-  // shape and buffers they were captured with; graphs_ok turns off after a
-  // failed capture
-  struct Graph {
-    hipGraphExec_t exec = nullptr;
-    int shape[5] = {0, 0, 0, 0, 0};
-    const void *ptrs[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  } graphs[17];
-  bool graphs_ok = true;
+  DevBuf<int> done_d;  // launch_small's workgroup counter, zero between launches
   DevBuf<double> bmax;
   // problem descriptor
   ProbDev prob{};
@@ -278,8 +270,6 @@ struct alpsg_ctx {
     DevBuf<double> *all[] = {&pperp, &ppar, &f0, &df1, &df2, &qs_d, &ms_d, &int_ee, &fitc, &polyc,
                              &bmax};
     for (auto *b : all) b->release();
-    for (auto &g : graphs)
-      if (g.exec) (void)hipGraphExecDestroy(g.exec);
     for (auto &g : osc_graphs)
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
     osc_d.release();
@@ -287,6 +277,7 @@ struct alpsg_ctx {
     if (oscctl_pin) (void)hipHostFree(oscctl_pin);
     work_d.release();
     zidx.release();
+    done_d.release();
     mcal_d.release();
     mval_d.release();
     mhit_d.release();
@@ -427,6 +418,13 @@ bool shape_is_valid(const int *t) {
   for (auto &v : kSweepVariants) a = a || (v[0] == t[0] && v[1] == t[1]);
   for (int v : kResonantLanes) b = b || (v == t[3]);
   return a && b && t[2] >= 1 && t[2] <= 64 && t[4] >= 1 && t[4] <= 16 && t[1] * t[2] <= 128;
+}
+
+// launch_small's workgroup counter (the stream's launches share it one after another)
+hipError_t ensure_done(alpsg_ctx *h) {
+  if (h->done_d.p) return hipSuccess;
+  const hipError_t e = h->done_d.ensure(1);
+  return e != hipSuccess ? e : hipMemsetAsync(h->done_d.p, 0, sizeof(int), h->st);
 }
 
 // The split-form tables of the current k (13 us of launches a species, which a
@@ -822,16 +820,12 @@ int autotune(alpsg_ctx *h, int n, const double2 *om_host, int *shape_out) {
 }
 
 // det D of a small batch (n <= REQ_MAX_N, det only, no closed-form or
-// relativistic species) by replaying the captured chain pinned copy in ->
-// k_sweep_req -> k_resonant parts -> k_assemble -> pinned copy out.  Returns
-// 1 when the chain cannot be captured (the caller then runs it eagerly).
-int graph_disp(alpsg_ctx *h, int n, const double *om, double *det) {
+// relativistic species) in one launch, which reads om from the pinned staging
+// and writes det there: two copies, three kernels and the gaps between them, as
+// a captured graph, took 53 us a call of one omega (two species of 50 x 100), this 33.
+int small_disp(alpsg_ctx *h, int n, const double *om, double *det) {
   const int ns = h->nspec;
   LaunchShape sh = shape_for(h, n);
-  const int shp[5] = {sh.nch_a, sh.w_a, sh.rc_a, sh.nch_b, sh.rb};
-  // every buffer at its small-batch size before a capture (no allocation inside)
-  HIPCHK(h->om_d.ensure(REQ_MAX_N));
-  HIPCHK(h->det_d.ensure(REQ_MAX_N));
   HIPCHK(h->chiA_d.ensure((size_t)REQ_MAX_N * REQ_TW * ns * 6));
   HIPCHK(h->chiB_d.ensure((size_t)REQ_MAX_N * ns * 2 * 16 * 6));
   HIPCHK(h->om_pin.ensure(PIN_MAX));
@@ -840,49 +834,11 @@ int graph_disp(alpsg_ctx *h, int n, const double *om, double *det) {
     HIPCHK(h->zidx.ensure(REQ_MAX_N));
     HIPCHK(hipMemsetAsync(h->zidx.p, 0, sizeof(int) * REQ_MAX_N, h->st));
   }
-  const void *ptrs[6] = {h->om_d.p, h->det_d.p, h->chiA_d.p, h->chiB_d.p, h->prob_d.p, h->zidx.p};
-  alpsg_ctx::Graph &g = h->graphs[n];
-  bool same = g.exec != nullptr;
-  for (int k = 0; k < 5 && same; ++k) same = g.shape[k] == shp[k];
-  for (int k = 0; k < 6 && same; ++k) same = g.ptrs[k] == ptrs[k];
-  if (!same) {
-    if (g.exec) {
-      HIPCHK(hipStreamSynchronize(h->st));
-      (void)hipGraphExecDestroy(g.exec);
-      g.exec = nullptr;
-    }
-    HIPCHK(hipStreamSynchronize(h->st));
-    if (hipStreamBeginCapture(h->st, hipStreamCaptureModeThreadLocal) != hipSuccess) return 1;
-    hipError_t e = hipMemcpyAsync(h->om_d.p, h->om_pin.p, sizeof(double2) * n,
-                                  hipMemcpyHostToDevice, h->st);
-    if (e == hipSuccess)
-      e = launch_sweep_req(h->st, REQ_NCH, REQ_W, REQ_TW / REQ_W, REQ_K, h->prob_d.p, n, h->om_d.p,
-                           h->chiA_d.p, h->zidx.p, true);
-    if (e == hipSuccess)
-      e = launch_resonant_all(h->st, sh.nch_b, sh.rb, h->prob_d.p, ns, n, h->om_d.p, h->chiB_d.p,
-                              h->lgen);
-    if (e == hipSuccess)
-      e = launch_assemble(h->st, h->prob_d.p, ns, n, REQ_TW / REQ_W, sh.rb, h->om_d.p, nullptr, h->chiA_d.p,
-                          h->chiB_d.p, nullptr, nullptr, nullptr, 0, nullptr, 0, h->det_d.p, nullptr,
-                          nullptr, nullptr);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(h->det_pin.p, h->det_d.p, sizeof(double2) * n, hipMemcpyDeviceToHost,
-                         h->st);
-    hipGraph_t graph = nullptr;
-    const hipError_t e2 = hipStreamEndCapture(h->st, &graph);
-    hipGraphExec_t exec = nullptr;
-    if (e == hipSuccess && e2 == hipSuccess && graph != nullptr &&
-        hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess) {
-      g.exec = exec;
-      for (int k = 0; k < 5; ++k) g.shape[k] = shp[k];
-      for (int k = 0; k < 6; ++k) g.ptrs[k] = ptrs[k];
-    }
-    if (graph) (void)hipGraphDestroy(graph);
-    (void)hipGetLastError();
-    if (!g.exec) return 1;
-  }
+  HIPCHK(ensure_done(h));
   std::memcpy(h->om_pin.p, om, sizeof(double2) * n);
-  HIPCHK(hipGraphLaunch(g.exec, h->st));
+  HIPCHK(launch_small(h->st, sh.nch_b, sh.rb, REQ_TW / REQ_W, h->prob_d.p, ns, n, h->om_pin.p,
+                      h->chiA_d.p, h->chiB_d.p, h->det_pin.p, h->zidx.p, h->lgen, h->done_d.p,
+                      nullptr, nullptr));
   HIPCHK(hipEventRecord(h->ev_done, h->st));
   hipError_t q;
   while ((q = hipEventQuery(h->ev_done)) == hipErrorNotReady) {
@@ -898,11 +854,8 @@ int run_disp(alpsg_ctx *h, int n, const double *om, double *det, double *chi, do
   if (!h->have_k) return fail(ALPSG_E_STATE, "alpsg_set_k has not been called");
   if (n < 0) return fail(ALPSG_E_ARG, "negative batch size");
   if (n == 0) return ALPSG_OK;
-  if (h->graphs_ok && n <= REQ_MAX_N && !chi && !low && !wave && !h->any_bm && !h->any_rel) {
-    const int rc = graph_disp(h, n, om, det);
-    if (rc != 1) return rc;
-    h->graphs_ok = false;  // capture is not available: run eagerly from now on
-  }
+  if (n <= REQ_MAX_N && !chi && !low && !wave && !h->any_bm && !h->any_rel)
+    return small_disp(h, n, om, det);
   HIPCHK(h->om_d.ensure(n));
   const bool pin = n <= PIN_MAX;
   if (pin) {
@@ -983,7 +936,7 @@ const int OSC_MAX_N = 1024;  // solves of one device-round batch (one workgroup 
 // run on the device (then cleared)
 int osc_graph_batch(alpsg_ctx *h, const alpsg_root_params *rp, int n, cplx *om, cplx *Dfin,
                     int *iters, std::function<int()> *work) {
-  if (!h->graphs_ok || !h->osc_graphs_ok || h->any_bm || h->any_rel || n > OSC_MAX_N) return -1;
+  if (!h->osc_graphs_ok || h->any_bm || h->any_rel || n > OSC_MAX_N) return -1;
   const int ns = h->nspec;
   LaunchShape sh = shape_for(h, n);
   const bool req = n <= REQ_MAX_N;
@@ -999,6 +952,7 @@ int osc_graph_batch(alpsg_ctx *h, const alpsg_root_params *rp, int n, cplx *om, 
     HIPCHK(h->zidx.ensure(REQ_MAX_N));
     HIPCHK(hipMemsetAsync(h->zidx.p, 0, sizeof(int) * REQ_MAX_N, h->st));
   }
+  HIPCHK(ensure_done(h));
   HIPCHK(h->osc_d.ensure(n));
   HIPCHK(h->oscctl_d.ensure(2));
   if (!h->oscctl_pin)
@@ -1044,9 +998,9 @@ int osc_graph_batch(alpsg_ctx *h, const alpsg_root_params *rp, int n, cplx *om, 
     hipError_t e = hipSuccess;
     for (int k = 0; k < OSC_K && e == hipSuccess; ++k) {
       if (req && REQ_W == 4 && REQ_NCH == 32 && REQ_K == 4) {
-        // the whole round in two launches
-        e = launch_round(h->st, sh.nch_b, sh.rb, REQ_TW / REQ_W, h->prob_d.p, ns, n, h->om_d.p,
-                         h->chiA_d.p, h->chiB_d.p, h->det_d.p, h->zidx.p, h->lgen,
+        // the whole round in one launch
+        e = launch_small(h->st, sh.nch_b, sh.rb, REQ_TW / REQ_W, h->prob_d.p, ns, n, h->om_d.p,
+                         h->chiA_d.p, h->chiB_d.p, h->det_d.p, h->zidx.p, h->lgen, h->done_d.p,
                          h->osc_d.p, h->oscctl_d.p);
         continue;
       }

@@ -1815,7 +1815,7 @@ __device__ __forceinline__ void assemble_block(
     const double2 *__restrict__ chiR, int RR, const double2 *__restrict__ lowR, int LR,
     double2 *__restrict__ det_out, double2 *__restrict__ chi_out, double2 *__restrict__ low_out,
     double2 *__restrict__ wave_out, int nspec, const int *__restrict__ pidx,
-    double2 *det_lds = nullptr) {
+    double2 *det_lds = nullptr, const double2 *stage = nullptr) {
   __shared__ double2 lchi[256];
   const int per = 6 * nspec;
   const int opb = 256 / per;  // omegas per block
@@ -1825,11 +1825,22 @@ __device__ __forceinline__ void assemble_block(
   const int iom = blk * opb + lo_om;
   const bool in = (lo_om < opb) && (iom < nom) && (active == nullptr || active[iom] != 0);
   const ProbDev &Pd = pidx != nullptr ? probp[pidx[min(iom, nom - 1)]] : *probp;
+  // (loaded beside the partial sums, not after them)
+  const double2 ov = in ? om_in[iom] : make_double2(0.0, 0.0);
   if (in) {
+    const SpecDev &S = Pd.sp[s];
+    const double ee = Pd.kperp_norm ? S.int_ee : Pd.kperp * Pd.kperp * S.int_ee;
+    const double norm = S.dens * S.q;
     // partial sums, loads issued in batches of 16
     cd v = mk(0.0, 0.0);
     const int tot = W + 2 * RB;
-    for (int base = 0; base < tot; base += 16) {
+    if (stage != nullptr)
+#pragma unroll 16
+      for (int j = 0; j < tot; ++j) {
+        const double2 a = stage[(size_t)(j * per + sk) * nom + iom];
+        v = v + mk(a.x, a.y);
+      }
+    for (int base = stage != nullptr ? tot : 0; base < tot; base += 16) {
       double2 buf[16];
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
@@ -1879,14 +1890,10 @@ __device__ __forceinline__ void assemble_block(
     // chi_sk with the ee term and the normalisation; this thread also writes
     // its mode's entries of the tensors (one thread per omega doing all of them
     // took 60 us of a 45-omega batch)
-    const SpecDev &S = Pd.sp[s];
-    const double ee = Pd.kperp_norm ? S.int_ee : Pd.kperp * Pd.kperp * S.int_ee;
     if (k == 2) v = v + mk(ee, 0.0);
-    const double norm = S.dens * S.q;
     v = v * norm;
     lchi[t] = make_double2(v.re, v.im);
     if (chi_out != nullptr || low_out != nullptr) {
-      const double2 ov = om_in[iom];
       const cd om = mk(ov.x, ov.y);
       cd dn = (om * om) * (Pd.vA * Pd.vA);
       if (!Pd.kperp_norm) dn = dn * (Pd.kperp * Pd.kperp);
@@ -1929,7 +1936,6 @@ __device__ __forceinline__ void assemble_block(
   }
   __syncthreads();
   if (!in || sk != 0) return;
-  const double2 ov = om_in[iom];
   const cd om = mk(ov.x, ov.y);
   cd eps[6];
   for (int q = 0; q < 6; ++q) eps[q] = mk(0.0, 0.0);
@@ -2246,11 +2252,11 @@ __global__ __launch_bounds__(1024) void k_osc_round(int n, alpsg_osc::OscMachine
 // Each thread's solve state is loaded first, beside the count of unfinished
 // solves, and det D reaches the step through LDS, so that the round waits on
 // global memory for the partial sums only.
-__global__ __launch_bounds__(256) void k_assemble_osc(
+__device__ __forceinline__ void assemble_osc(
     const ProbDev *__restrict__ probp, int nom, int W, int RB, const double2 *__restrict__ om_in,
     const double2 *__restrict__ chiA, const double2 *__restrict__ chiB, double2 *__restrict__ det,
     int nspec, alpsg_osc::OscMachine *__restrict__ S, double2 *__restrict__ om_next,
-    int *__restrict__ round_ctr, int *__restrict__ remaining) {
+    int *__restrict__ round_ctr, int *__restrict__ remaining, const double2 *stage = nullptr) {
   __shared__ double2 det_l[256];
   const int t = threadIdx.x;
   alpsg_osc::OscMachine m;
@@ -2263,7 +2269,7 @@ __global__ __launch_bounds__(256) void k_assemble_osc(
   const int opb = 256 / (6 * nspec);
   for (int blk = 0; blk * opb < nom; ++blk) {
     assemble_block(blk, probp, nom, W, RB, om_in, nullptr, chiA, chiB, nullptr, nullptr, nullptr, 0,
-                   nullptr, 0, det, nullptr, nullptr, nullptr, nspec, nullptr, det_l);
+                   nullptr, 0, det, nullptr, nullptr, nullptr, nspec, nullptr, det_l, stage);
     __syncthreads();
   }
   int more = 0;
@@ -2285,78 +2291,130 @@ __global__ __launch_bounds__(256) void k_assemble_osc(
   }
 }
 
-// The request sweep and both resonant parts of a small batch in one launch:
-// workgroups [0, nom RC) run the sweep (omega b % nom, workgroup b / nom of
-// RC), the others four resonant wavefronts each (every part and harmonic
-// block).
-template <int NCHS, int K, int NCHR, int GEN>
-__global__ __launch_bounds__(256) void k_sweep_res(const ProbDev *__restrict__ probp, int nom,
-                                                   const double2 *__restrict__ om,
-                                                   double2 *__restrict__ chiA,
-                                                   double2 *__restrict__ chiB,
-                                                   const int *__restrict__ zidx, int RC, int RB,
-                                                   int nspec, const int *__restrict__ remaining) {
+__global__ __launch_bounds__(256) void k_assemble_osc(
+    const ProbDev *__restrict__ probp, int nom, int W, int RB, const double2 *__restrict__ om_in,
+    const double2 *__restrict__ chiA, const double2 *__restrict__ chiB, double2 *__restrict__ det,
+    int nspec, alpsg_osc::OscMachine *__restrict__ S, double2 *__restrict__ om_next,
+    int *__restrict__ round_ctr, int *__restrict__ remaining) {
+  assemble_osc(probp, nom, W, RB, om_in, chiA, chiB, det, nspec, S, om_next, round_ctr, remaining);
+}
+
+// A small batch in one launch.  Workgroups [0, nom RC) run the request sweep
+// (omega b % nom, workgroup b / nom of RC; 32 lanes per row pair, 4 records in
+// flight), the others four resonant wavefronts each (every part and harmonic
+// block).  The workgroup that finishes last assembles det D of every omega and,
+// with OSC, feeds it to the solves: a launch of its own for that costs its
+// start and end, and every one of them writes back and refills what it shares
+// with the next.  Each workgroup's partial sums are released to the device
+// before it counts itself in done; the last one acquires them, and sets done
+// back to zero for the next launch (a secant round of one root, two species of
+// 50 x 100: 11.1 + 6.2 us and the gap between two launches, 15.1 us so).
+// om and det may lie in host memory that the device can reach.
+constexpr int SMALL_STAGE = 1024;
+template <int NCHR, int GEN, bool OSC>
+__global__ __launch_bounds__(256) void k_small(const ProbDev *__restrict__ probp, int nom,
+                                               double2 *om, double2 *chiA, double2 *chiB,
+                                               const int *__restrict__ zidx, int RC, int RB,
+                                               int nspec, double2 *det, int *done,
+                                               alpsg_osc::OscMachine *S, int *ctl) {
   constexpr int OMB = 64 / NCHR;
   __shared__ double win[4][OMB * 2 * PV_WIN];
-  if (*remaining == 0) return;  // every solve has finished: nothing to evaluate
+  __shared__ int last;
+  if constexpr (OSC)
+    if (ctl[1] == 0) return;  // every solve has finished: nothing to evaluate
   const int A = nom * RC;
   const int b = blockIdx.x;
-  if (b < A) {
-    sweep_req_body<NCHS, 4, K, true>(probp, nom, om, chiA, zidx, b % nom, b / nom, RC);
-    return;
-  }
   const int gx = (nom + OMB - 1) / OMB;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int vb = (b - A) * 4 + wave;
-  if (vb >= gx * nspec * 2 * RB) return;
-  const int x = vb % gx, y = (vb / gx) % nspec, z = vb / (gx * nspec);
-  if (z < RB) {
-    resonant_body<NCHR, 0>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z, x, y, lane,
-                           win[wave]);
-    return;
+  if (b < A) {
+    sweep_req_body<32, 4, 4, true>(probp, nom, om, chiA, zidx, b % nom, b / nom, RC);
+  } else if (vb < gx * nspec * 2 * RB) {
+    const int x = vb % gx, y = (vb / gx) % nspec, z = vb / (gx * nspec);
+    if (z < RB) {
+      resonant_body<NCHR, 0>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z, x, y, lane,
+                             win[wave]);
+    } else {
+      resonant_body<NCHR, 1>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y,
+                             lane, win[wave]);
+      if constexpr ((GEN & 1) != 0)
+        resonant_body<NCHR, 2>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y,
+                               lane, win[wave]);
+      if constexpr ((GEN & 2) != 0)
+        resonant_body<NCHR, 3>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y,
+                               lane, win[wave]);
+    }
   }
-  resonant_body<NCHR, 1>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y, lane,
-                         win[wave]);
-  if constexpr ((GEN & 1) != 0)
-    resonant_body<NCHR, 2>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y, lane,
-                           win[wave]);
-  if constexpr ((GEN & 2) != 0)
-    resonant_body<NCHR, 3>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y, lane,
-                           win[wave]);
+  // every wavefront's stores are acknowledged, then one lane releases them all
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+           (int)gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  if (threadIdx.x == 0) *done = 0;
+  // the partial sums of a few omegas through LDS, every one in flight at once
+  // (they are summed in the same order)
+  __shared__ double2 sums[SMALL_STAGE];
+  const int na = nom * 6 * nspec * RC, nb = nom * 6 * nspec * 2 * RB;
+  const double2 *stage = na + nb <= SMALL_STAGE ? sums : nullptr;
+  if (stage != nullptr) {
+    constexpr int U = SMALL_STAGE / 256;
+    double2 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = threadIdx.x + 256 * u;
+      if (i < na + nb) v[u] = i < na ? chiA[i] : chiB[i - na];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if ((int)threadIdx.x + 256 * u < na + nb) sums[threadIdx.x + 256 * u] = v[u];
+    __syncthreads();
+  }
+  if constexpr (OSC) {
+    assemble_osc(probp, nom, RC, RB, om, chiA, chiB, det, nspec, S, om, ctl, ctl + 1, stage);
+  } else {
+    const int opb = 256 / (6 * nspec);
+    for (int blk = 0; blk * opb < nom; ++blk) {
+      assemble_block(blk, probp, nom, RC, RB, om, nullptr, chiA, chiB, nullptr, nullptr, nullptr, 0,
+                     nullptr, 0, det, nullptr, nullptr, nullptr, nspec, nullptr, nullptr, stage);
+      __syncthreads();
+    }
+  }
 }
 
 }  // namespace
 
-// a secant round of a small batch in two launches: the request sweep (32
-// lanes per row pair, 4 records in flight, 4 wavefronts per workgroup, RC
-// workgroups per omega) with both resonant parts (nchr lanes per omega, RB
-// harmonic blocks), then the assembly and the secant step in one workgroup;
-// ctl = {round, unfinished}
-hipError_t launch_round(hipStream_t st, int nchr, int RB, int RC, const ProbDev *prob, int nspec,
+// det D of a small batch, and with S one secant step of its solves (om is then
+// overwritten with the next frequencies; ctl = {round, unfinished}): nchr lanes
+// per omega and RB harmonic blocks in the resonant parts, RC sweep workgroups
+// per omega; done: a counter that is zero between launches
+hipError_t launch_small(hipStream_t st, int nchr, int RB, int RC, const ProbDev *prob, int nspec,
                         int nom, double2 *om, double2 *chiA, double2 *chiB, double2 *det,
-                        const int *zidx, int lgen, alpsg_osc::OscMachine *S, int *ctl) {
+                        const int *zidx, int lgen, int *done, alpsg_osc::OscMachine *S, int *ctl) {
   if (nom <= 0) return hipSuccess;
-  if (nom > 256 || 6 * nspec > 256) return hipErrorInvalidValue;
-  bool ok = false;
+  if (nom > 256 || 6 * nspec > 256 || lgen < 0 || lgen > 3) return hipErrorInvalidValue;
 #define RDG(N, G)                                                                                  \
-  if (lgen == G)                                                                                   \
-    hipLaunchKernelGGL((k_sweep_res<32, 4, N, G>), dim3(grid), dim3(256), 0, st, prob, nom, om,    \
-                       chiA, chiB, zidx, RC, RB, nspec, ctl + 1);
+  if (lgen == G) {                                                                                 \
+    if (S != nullptr)                                                                              \
+      hipLaunchKernelGGL((k_small<N, G, true>), dim3(grid), dim3(256), 0, st, prob, nom, om, chiA, \
+                         chiB, zidx, RC, RB, nspec, det, done, S, ctl);                            \
+    else                                                                                           \
+      hipLaunchKernelGGL((k_small<N, G, false>), dim3(grid), dim3(256), 0, st, prob, nom, om,      \
+                         chiA, chiB, zidx, RC, RB, nspec, det, done, S, ctl);                      \
+  }
 #define RD(N)                                                                                      \
   if (nchr == N) {                                                                                 \
     const int gx = (nom + (64 / N) - 1) / (64 / N);                                                \
     const int grid = nom * RC + (gx * nspec * 2 * RB + 3) / 4;                                     \
     RDG(N, 0) RDG(N, 1) RDG(N, 2) RDG(N, 3)                                                        \
-    ok = true;                                                                                     \
+    return hipGetLastError();                                                                      \
   }
-  if (lgen < 0 || lgen > 3) return hipErrorInvalidValue;
   RD(4) RD(8) RD(16) RD(32) RD(64)
 #undef RD
 #undef RDG
-  if (!ok) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_assemble_osc, dim3(1), dim3(256), 0, st, prob, nom, RC, RB, om, chiA, chiB,
-                     det, nspec, S, om, ctl, ctl + 1);
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_resonant_all(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec,
