@@ -1392,6 +1392,17 @@ __device__ void landau_part(const SpecDev &S, const ProbDev &Pd, int an, const R
     // evaluations instead of four (the same values and the same row
     // formulas), made one at a time (unroll 1: their temporaries are not live
     // together)
+    // a zero of one row makes the whole term zero, and the row of the largest
+    // pperp, where f0 is smallest, is the one that underflows or is clipped first:
+    // its three values come first, a lane each, and a zero ends the term there
+    // (a 96 x 64 map of a Chebyshev continuation: 331 us of these sums, 236 so)
+    static_assert(NCH >= 3, "a lane for each value of the last tested row");
+    cd last = mk(1.0, 0.0);
+    if (c < 3) last = F(c == 2 ? nperp : nperp - 1, c == 0 ? 1 : (c == 1 ? -1 : 0));
+    if (gor<NCH>(czero(last) ? 1 : 0)) {
+      zero = 1;
+      return;
+    }
     const int blk = (nperp + 1 + NCH - 1) / NCH;
     const int r0 = c * blk, r1 = min(r0 + blk, nperp + 1) - 1;
     if (r0 > r1) return;
