@@ -64,7 +64,8 @@ hipError_t launch_map_grid(hipStream_t st, int nr, int ni, double omi, double dr
 hipError_t launch_osc_round(hipStream_t st, int n, alpsg_osc::OscMachine *S, const double2 *det,
                             double2 *om, int *round_ctr, int *remaining);
 hipError_t launch_resonant_all(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec,
-                               int nom, const double2 *om, double2 *chiB, int lgen);
+                               int nom, const double2 *om, double2 *chiB, int lgen,
+                               const int *pidx = nullptr);
 hipError_t launch_small(hipStream_t st, int nchr, int RB, int RC, const ProbDev *prob, int nspec,
                         int nom, double2 *om, double2 *chiA, double2 *chiB, double2 *det,
                         const int *zidx, int lgen, int *done, alpsg_osc::OscMachine *S, int *ctl);

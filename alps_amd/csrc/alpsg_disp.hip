@@ -1795,20 +1795,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 template <int NCH, int GEN>
 __global__ __launch_bounds__(64) void k_resonant_all(const ProbDev *__restrict__ probp, int nom,
                                                      const double2 *__restrict__ om_in,
-                                                     double2 *__restrict__ chiB, int RB) {
+                                                     double2 *__restrict__ chiB,
+                                                     const int *__restrict__ pidx, int RB) {
   __shared__ double win[(64 / NCH) * 2 * PV_WIN];
   const int z = blockIdx.z, bx = blockIdx.x, by = blockIdx.y, lane = threadIdx.x;
   if (z < RB) {
-    resonant_body<NCH, 0>(probp, nom, om_in, nullptr, chiB, nullptr, nullptr, RB, z, bx, by, lane, win);
+    resonant_body<NCH, 0>(probp, nom, om_in, nullptr, chiB, nullptr, pidx, RB, z, bx, by, lane, win);
     return;
   }
-  resonant_body<NCH, 1>(probp, nom, om_in, nullptr, chiB, nullptr, nullptr, RB, z - RB, bx, by, lane,
+  resonant_body<NCH, 1>(probp, nom, om_in, nullptr, chiB, nullptr, pidx, RB, z - RB, bx, by, lane,
                         win);
   if constexpr ((GEN & 1) != 0)
-    resonant_body<NCH, 2>(probp, nom, om_in, nullptr, chiB, nullptr, nullptr, RB, z - RB, bx, by,
+    resonant_body<NCH, 2>(probp, nom, om_in, nullptr, chiB, nullptr, pidx, RB, z - RB, bx, by,
                           lane, win);
   if constexpr ((GEN & 2) != 0)
-    resonant_body<NCH, 3>(probp, nom, om_in, nullptr, chiB, nullptr, nullptr, RB, z - RB, bx, by,
+    resonant_body<NCH, 3>(probp, nom, om_in, nullptr, chiB, nullptr, pidx, RB, z - RB, bx, by,
                           lane, win);
 }
 
@@ -2429,13 +2430,15 @@ hipError_t launch_small(hipStream_t st, int nchr, int RB, int RC, const ProbDev 
 }
 
 hipError_t launch_resonant_all(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec,
-                               int nom, const double2 *om, double2 *chiB, int lgen) {
+                               int nom, const double2 *om, double2 *chiB, int lgen,
+                               const int *pidx) {
   if (nom <= 0) return hipSuccess;
+  if (pidx != nullptr && nch != 64) return hipErrorInvalidValue;
   if (lgen < 0 || lgen > 3) return hipErrorInvalidValue;
 #define RAG(N, G)                                                                              \
   if (lgen == G)                                                                               \
     hipLaunchKernelGGL((k_resonant_all<N, G>), dim3(grid, nspec, 2 * RB), dim3(64), 0, st,     \
-                       prob, nom, om, chiB, RB);
+                       prob, nom, om, chiB, pidx, RB);
 #define RA(N)                                                                                  \
   if (nch == N) {                                                                              \
     const int grid = (nom + (64 / N) - 1) / (64 / N);                                          \

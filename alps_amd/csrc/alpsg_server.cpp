@@ -76,6 +76,9 @@ hipError_t launch_sweep_req(hipStream_t st, int nch, int W, int RC, int K, const
 hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec, int nom,
                            const double2 *om, const int *active, double2 *chiB, double2 *lowB,
                            int lgen, const int *pidx, int P, const LandTabs *tabs = nullptr);
+hipError_t launch_resonant_all(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec,
+                               int nom, const double2 *om, double2 *chiB, int lgen,
+                               const int *pidx);
 hipError_t launch_assemble(hipStream_t st, const ProbDev *prob, int nspec, int nom, int W, int RB,
                            const double2 *om, const int *active, const double2 *chiA,
                            const double2 *chiB, const double2 *lowA, const double2 *lowB,
@@ -1099,8 +1102,15 @@ int server_pass(alpsg_server *S) {
       SCHK(launch_sweep_req(S->st, SW_NCH, SW_W, SW_RC, SW_K, S->probs_d, n, S->om_d + i0,
                             S->chiA, S->pidx_d + i0, false));
       if (ev) SCHK(hipEventRecord(ev[1], S->st));
-      SCHK(launch_resonant(S->st, 64, RS_RB, S->probs_d, ns, n, S->om_d + i0, nullptr, S->chiB,
-                           nullptr, gen, S->pidx_d + i0, 0));
+      // both resonant parts in one launch (512 requests: 15 + 10 us a pass, 18 so);
+      // the general Landau forms keep launches of their own, with the registers and
+      // wavefronts that suit each
+      if (gen == 0)
+        SCHK(launch_resonant_all(S->st, 64, RS_RB, S->probs_d, ns, n, S->om_d + i0, S->chiB, gen,
+                                 S->pidx_d + i0));
+      else
+        SCHK(launch_resonant(S->st, 64, RS_RB, S->probs_d, ns, n, S->om_d + i0, nullptr, S->chiB,
+                             nullptr, gen, S->pidx_d + i0, 0));
       // closed-form species: partial slot 0 of their chi (the sweep left it zero)
       if (bm)
         SCHK(launch_nhds(S->st, S->probs_d, ns, n, S->om_d + i0, nullptr, S->chiA, nullptr,
