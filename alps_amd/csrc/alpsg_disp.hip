@@ -2321,10 +2321,12 @@ __global__ __launch_bounds__(256) void k_assemble_osc(
 // before it counts itself in done; the last one acquires them, and sets done
 // back to zero for the next launch (a secant round of one root, two species of
 // 50 x 100: 11.1 + 6.2 us and the gap between two launches, 15.1 us so).
-// om and det may lie in host memory that the device can reach.
+// om and det may lie in host memory that the device can reach.  Held to two
+// wavefronts per SIMD: 16 omegas of three species are two workgroups a CU (their
+// rounds 57 us at one, 49 at two).
 constexpr int SMALL_STAGE = 1024;
 template <int NCHR, int GEN, bool OSC>
-__global__ __launch_bounds__(256) void k_small(const ProbDev *__restrict__ probp, int nom,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_small(const ProbDev *__restrict__ probp, int nom,
                                                double2 *om, double2 *chiA, double2 *chiB,
                                                const int *__restrict__ zidx, int RC, int RB,
                                                int nspec, double2 *det, int *done,
