@@ -732,7 +732,10 @@ __global__ __launch_bounds__(64 * RSW) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int it0 = 0; it0 < 4 * NC; it0 += 64) {
           const int it = min(it0 + lane, 4 * NC - 1);
           const int g = it / NC, ci = it - g * NC, src = 2 * r + g;
-          const bool on = it0 + lane < 4 * NC && __shfl(R.pv, src, 64) == 1;
+          // (every lane takes part in the shuffles, also those past the last item:
+          // the rows they hold are other lanes' sources)
+          const int pvs = __shfl(R.pv, src, 64);
+          const bool on = it0 + lane < 4 * NC && pvs == 1;
           RelLadder L;
           L.dR = __shfl(R.dR, src, 64);
           L.cap = __shfl(R.cap, src, 64);

@@ -1,6 +1,7 @@
 """The relativistic kernels of a frequency batch where their split and their
-ladder cells can go wrong: batch sizes on both sides of each split, the largest
-principal-value window, odd grids, and (Gamma, pparbar) tables whose rows are not
+ladder cells can go wrong: batch sizes on both sides of each split, as many Gamma
+rows as a wavefront takes at once and more, the smallest and the largest
+principal-value windows, odd grids, and (Gamma, pparbar) tables whose rows are not
 the same grid (a row's ladder then leaves the cells around its resonance).
 
 Bar: 1e-11 of the largest |chi| of the species (tests/test_gpu_disp.py), or ten
@@ -12,6 +13,7 @@ import numpy as np
 import pytest
 
 import cases
+from alps_amd.plasma import juttner_plasma
 from oracle import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -59,6 +61,23 @@ def test_window_sizes(pos, npparbar):
     p = dataclasses.replace(cases.rel_pair(nperp=12, npar=41, ngamma=21, npparbar=npparbar),
                             positions_principal=pos)
     _check(p, 0.31, 0.29, OMS)
+
+
+@pytest.mark.parametrize("ngamma,pos,sizes", [
+    (100, 3, (256, 257, 300)), (200, 3, (64, 65, 256, 257)), (400, 3, (1, 64)),
+    (100, 1, (300,)), (100, 2, (300,)), (150, 4, (300,)), (100, 5, (300,)),
+    (100, 6, (1, 65, 257)), (150, 7, (1, 257)), (100, 10, (1, 65, 300))])
+def test_many_gamma_rows(ngamma, pos, sizes):
+    """All 32 Gamma rows that a wavefront of k_rel_res decides at once, and a second
+    32 of them (200 rows at 257 omegas), for windows of fewer and of more cells than
+    it has lanes.  The omegas' n = 0 resonances lie inside the cone on every row
+    from the first few on."""
+    p = juttner_plasma(ms=[1.0, 1.0], qs=[1.0, -1.0], ns=[1.0, 1.0], taus=[1.0, 1.0], beta=1.0,
+                       vA=1.0, nperp=12, npar=24 if pos < 10 else 41, maxP=5.0, ngamma=ngamma,
+                       npparbar=400 if pos > 5 else 200, analytic_rel=True,
+                       positions_principal=pos, n_resonance_interval=100, Tlim=0.01,
+                       Bessel_zero=1e-45)
+    _check(p, 0.3, 0.3, [0.1217 + 0.03j, 0.2113 + 0.0011j, 0.1531 - 0.004j], sizes=sizes)
 
 
 def test_rows_on_grids_of_their_own():
