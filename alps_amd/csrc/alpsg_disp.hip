@@ -1479,18 +1479,21 @@ __device__ void landau_part(const SpecDev &S, const ProbDev &Pd, int an, const R
 namespace {
 
 // harmonics nlo..nhi whose p_res = (m w - n q)/kpar can satisfy determine_resonances:
-// Re p_res in [pa[1] - P dppar, max(pa[npar], pa[npar-1] + P dppar)), widened by one
+// Re p_res in [pa[1] - P dppar, max(pa[npar], pa[npar-1] + P dppar)), widened by one.
+// Both ends stay within one of +-nmax: an omega far off the grid gives no harmonics,
+// and not an end at the largest int, past which nlo + rb wraps round
 __device__ __forceinline__ void res_harmonics(const SpecDev &S, int P, double kpar, double omr,
                                               bool valid, int &nlo, int &nhi) {
   nlo = 1;
   nhi = 0;
-  if (!valid || omr != omr) return;
+  if (!valid || omr != omr || S.nmax < 0) return;  // (nmax < 0: a species without node tables)
   const double L = S.ppar[1] - P * S.dppar;
   const double U = fmax(S.ppar[S.npar], S.ppar[S.npar - 1] + P * S.dppar);
   const double n1 = (S.m * omr - kpar * L) / S.q, n2 = (S.m * omr - kpar * U) / S.q;
   const double lo_d = fmin(n1, n2) - 1.0, hi_d = fmax(n1, n2) + 1.0;
-  nlo = (int)fmax(floor(lo_d), -(double)S.nmax);
-  nhi = (int)fmin(ceil(hi_d), (double)S.nmax);
+  const double nm = (double)S.nmax;
+  nlo = (int)fmin(fmax(floor(lo_d), -nm), nm + 1.0);
+  nhi = (int)fmax(fmin(ceil(hi_d), nm), -nm - 1.0);
 }
 
 // the modes of harmonic n's Landau term from its pperp sums (int_T_res,

@@ -58,6 +58,27 @@ def test_branches_drift_aniso():
     _check(p, 0.3, 0.3, cases.BRANCH_OMEGAS)
 
 
+@pytest.mark.parametrize("case", ["small_bimax", "kappa_case", "poly_case"])
+@pytest.mark.parametrize("n", [4, 40, 600, 1100])
+def test_omegas_far_off_the_grid(case, n):
+    """No harmonic of an omega beyond 2^31 q/m resonates: the harmonic range of the
+    resonant parts is empty there, whatever the sign of omega and of the charge."""
+    p = getattr(cases, case)()
+    oms = [0.4 - 0.01j, 2e9 + 1e8j, -3e9 - 1e8j, 5e12 + 1j, 1e20 + 1e19j, -1e30 - 1e29j]
+    O, E = Oracle(p), _engine(p)
+    assert O.set_k(0.3, 0.3) == E.set_k(0.3, 0.3)
+    det, chi, low, _ = E.disp_batch(np.resize(np.array(oms), n), want_tensors=True)
+    one = E.disp_batch(oms[:min(n, 6)])
+    for k in range(min(n, 6)):
+        d, c, lo, wave = O.disp(oms[k], want_tensors=True)
+        for s in range(p.nspec):
+            for g, o in ((chi[k, s], c[s]), (low[k, s], lo[s])):
+                assert np.max(np.abs(g - o)) <= TOL * np.max(np.abs(o)), (oms[k], s)
+        for g in (det[k], one[k]):
+            assert abs(g - d) <= TOL * cases.det_scale(wave), oms[k]
+    E.close()
+
+
 def test_three_species():
     p = cases.three_species()
     _check(p, 0.5, 0.2, cases.BRANCH_OMEGAS)
