@@ -241,11 +241,15 @@ __global__ __launch_bounds__(64 * NRW) __attribute__((amdgpu_waves_per_eu(4))) v
     if (low && threadIdx.x < 18) low[threadIdx.x] = make_double2(0.0, 0.0);
     return;
   }
-  const bool all4 = use[0] && use[1] && use[2] && use[3];
   const double2 ov = om_in[iom];
   const double omr = ov.x, omi = ov.y;
   const double m = S.m, q = S.q, kpar = Pd.kpar;
   const double nqa = (1.0 * na) * q, nqb = (1.0 * nb) * q;
+  // the one reciprocal needs the product of four |den|^2 to be a double: |den|
+  // below 1e38, of which an omega beyond about 1e37 is short (its sums are finite)
+  const double dmax = S.rel_gmax * m * (fabs(omr) + fabs(omi)) + fabs(nqb) +
+                      fabs(kpar) * fmax(fabs(S.ppar[0]), fabs(S.ppar[npar]));
+  const bool all4 = use[0] && use[1] && use[2] && use[3] && dmax < 1e38;
   typedef const __attribute__((address_space(4))) double *cptr;
   // (a pair past nmax is never used; its table pointer stays in range)
   const cptr ata = (cptr)(S.atab + (size_t)(na <= nmax ? na : 0) * (nperp + 1) * ATAB_STRIDE);

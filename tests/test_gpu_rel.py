@@ -47,6 +47,7 @@ def _check(p, kperp, kpar, oms, sizes=(None,)):
             for s in range(p.nspec):
                 for g, o, j in ((chi[k, s], c[s], jc[s]), (low[k, s], l[s], jl[s])):
                     sc = max(np.max(np.abs(o)), 1e-300)
+                    assert np.all(np.isfinite(g))
                     tol = max(TOL, 10.0 * np.max(j) / sc)
                     assert np.max(np.abs(g - o)) / sc <= tol, (n, k, om[k], s)
     E.close()
@@ -78,6 +79,13 @@ def test_many_gamma_rows(ngamma, pos, sizes):
                        positions_principal=pos, n_resonance_interval=100, Tlim=0.01,
                        Bessel_zero=1e-45)
     _check(p, 0.3, 0.3, [0.1217 + 0.03j, 0.2113 + 0.0011j, 0.1531 - 0.004j], sizes=sizes)
+
+
+def test_far_omegas():
+    """omegas whose |den|^2 of four harmonics have no product in double precision
+    (beyond 3e38), and one on the other side: D is finite up to 1e50"""
+    _check(cases.rel_pair(), 0.3, 0.3, [1e30 + 1e29j, 1e39 + 2e38j, 1e40 + 1e39j, 1e45 - 1e44j],
+           sizes=(4, 300))
 
 
 def test_rows_on_grids_of_their_own():
