@@ -2388,6 +2388,36 @@ int alpsg_sweep_work(alpsg_handle h, int n, const double *om, double *work3) {
   ALPSG_CATCH
 }
 
+int alpsg_landau_work(alpsg_handle h, int n, const double *om, double *work2) {
+  ALPSG_TRY
+  if (!h || !work2 || (n > 0 && !om)) return fail(ALPSG_E_ARG, "null argument");
+  if (!h->have_k) return fail(ALPSG_E_STATE, "alpsg_set_k has not been called");
+  if (n < 0) return fail(ALPSG_E_ARG, "negative batch size");
+  work2[0] = work2[1] = 0.0;
+  if (n == 0) return ALPSG_OK;
+  const LaunchShape sh = shape_for(h, n);
+  LandTabs tabs;
+  bool use = false;
+  if (const int rc = landau_tables(h, n, bounds_of(om, n), sh.rb, tabs, use)) return rc;
+  if (!use) return ALPSG_OK;
+  HIPCHK(h->om_d.ensure(n));
+  HIPCHK(h->chiB_d.ensure((size_t)n * h->nspec * 2 * sh.rb * 6));
+  HIPCHK(hipMemcpyAsync(h->om_d.p, om, sizeof(double2) * n, hipMemcpyHostToDevice, h->st));
+  HIPCHK(launch_resonant(h->st, sh.nch_b, sh.rb, h->prob_d.p, h->nspec, n, h->om_d.p, nullptr,
+                         h->chiB_d.p, nullptr, h->lgen, nullptr, h->P, &tabs));
+  const size_t per = (size_t)sh.rb * n;  // (species, harmonic block, omega)
+  std::vector<unsigned char> need((size_t)h->nspec * per);
+  HIPCHK(hipMemcpyAsync(need.data(), h->landneed.p, need.size(), hipMemcpyDeviceToHost, h->st));
+  HIPCHK(hipStreamSynchronize(h->st));
+  for (int s = 0; s < h->nspec; ++s) {
+    if (tabs.sp[s].c == nullptr) continue;  // (its part of need is not written)
+    work2[0] += 1.0;
+    for (size_t i = s * per; i < (s + 1) * per; ++i) work2[1] += need[i];
+  }
+  return ALPSG_OK;
+  ALPSG_CATCH
+}
+
 int alpsg_last_kernel_split(alpsg_handle h, double *ms3) {
   ALPSG_TRY
   if (!h || !ms3) return fail(ALPSG_E_ARG, "null argument");

@@ -47,7 +47,8 @@ EXPORTS = ["alpsg_last_error", "alpsg_create", "alpsg_destroy", "alpsg_set_k",
            "alpsg_server_submit", "alpsg_server_poll", "alpsg_server_stats",
            "alpsg_server_destroy", "alpsg_determine_param_fit", "alpsg_last_scan_steps",
            "alpsg_set_plain_roots", "alpsg_disp_batch_noalloc", "alpsg_server_work",
-           "alpsg_set_sweep_series", "alpsg_sweep_work", "alpsg_map_search_refine"]
+           "alpsg_set_sweep_series", "alpsg_sweep_work", "alpsg_map_search_refine",
+           "alpsg_landau_work"]
 
 
 class AlpsgError(RuntimeError):
@@ -140,6 +141,8 @@ def load_library(path: str = LIB_PATH):
     L.alpsg_set_sweep_series.restype = C.c_int
     L.alpsg_sweep_work.argtypes = [vp, C.c_int, dp, dp]
     L.alpsg_sweep_work.restype = C.c_int
+    L.alpsg_landau_work.argtypes = [vp, C.c_int, dp, dp]
+    L.alpsg_landau_work.restype = C.c_int
     L.alpsg_autotune.argtypes = [vp, C.c_int, dp, ip]
     L.alpsg_set_shape.argtypes = [vp, C.c_int, ip]
     L.alpsg_get_shape.argtypes = [vp, C.c_int, ip]
@@ -455,6 +458,15 @@ class Engine:
         out = np.zeros(3)
         _check(load_library().alpsg_sweep_work(self._h, om.size, _dp(om), _dp(out)))
         return tuple(float(x) for x in out)
+
+    def landau_work(self, om):
+        """What a batch of these omegas takes from Landau tables: (species with
+        tables, (species, harmonic block, omega) shares with a row left to the
+        row sums)."""
+        om = np.ascontiguousarray(np.asarray(om, dtype=np.complex128).ravel())
+        out = np.zeros(2)
+        _check(load_library().alpsg_landau_work(self._h, om.size, _dp(om), _dp(out)))
+        return tuple(int(x) for x in out)
 
     def refine_guess(self, guesses, roots: RootParams | None = None):
         """refine_guess (ALPS_fns.f90:3793-3856): secant on each guess, then det D there."""

@@ -301,6 +301,13 @@ int alpsg_set_sweep_series(alpsg_handle h, int on);
    summed over the omegas.  The sweep's partial results are discarded. */
 int alpsg_sweep_work(alpsg_handle h, int n, const double *om, double *work3);
 
+/* What a batch of these n omegas takes from Landau tables (the pperp sums of
+   landau_integrate, ALPS_fns.f90:1327-1452, tabulated for the batch):
+   work2[0] the species that get tables, work2[1] the (species, harmonic block,
+   omega) shares with a row that their tiles do not cover, which take the row
+   sums.  The partial results are discarded. */
+int alpsg_landau_work(alpsg_handle h, int n, const double *om, double *work2);
+
 /* Device time (ms) of the last alpsg_disp_batch / alpsg_map_search kernel
    sweep, measured with HIP events on the handle's stream. */
 double alpsg_last_kernel_ms(alpsg_handle h);

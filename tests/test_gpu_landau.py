@@ -1,7 +1,9 @@
 """The Landau tables of a frequency batch where they can go wrong: batch sizes on
 both sides of the rule that builds them, omegas at the tables' edges (real axis,
 last tile row, one row too deep), beside the continuation's branch points, with
-omegas that are NaN or have no Landau term, and the n = -1, 0, 1 parts.
+omegas that are NaN or have no Landau term, the most harmonics a table holds and
+one more, and the n = -1, 0, 1 parts.  Each case states how many species get
+tables, and most of what they cover has to come from them (alpsg_landau_work).
 
 Bar: a tile's series is held to 2^-51 of the sums of absolute values, so 1e-11 of
 the species' largest |chi| (tests/test_gpu_disp.py) leaves 2e4 for cancellation
@@ -21,13 +23,13 @@ TOL = 1e-11
 KPERP, KPAR = 0.3, 0.41
 
 
-def _tile(p, s):
+def _tile(p, s, kpar=KPAR):
     """side of a tile and the resonant harmonics of an omega (landau_tables)"""
     pa = p.pp[s, 2, :, 1]
     d = abs(pa[2] - pa[1])
     lo = pa[1] - p.positions_principal * d
     up = max(pa[-1], pa[-2] + p.positions_principal * d)
-    return (up - lo) * (1 + 1e-6) / 64, KPAR * (up - lo) / abs(p.qs[s]), lo, up
+    return (up - lo) * (1 + 1e-6) / 64, abs(kpar) * (up - lo) / abs(p.qs[s]), lo, up
 
 
 def _batch(p, n, depth, seed=5):
@@ -39,11 +41,13 @@ def _batch(p, n, depth, seed=5):
     return om
 
 
-def _compare(p, om, low=True):
+def _compare(p, om, tabs, kpar=KPAR):
     from alps_amd.engine import Engine
     E = Engine(p)
     O = Oracle(p)
-    assert E.set_k(KPERP, KPAR) == O.set_k(KPERP, KPAR)
+    assert E.set_k(KPERP, kpar) == O.set_k(KPERP, kpar)
+    got, left = E.landau_work(om)
+    assert got == tabs and left < 0.5 * max(tabs, 1) * len(om) * E.get_shape(len(om))[4]
     big = E.disp_batch(om, want_tensors=True)
     parts = [E.disp_batch(om[i:i + 200], want_tensors=True) for i in range(0, len(om), 200)]
     row = [np.concatenate([np.asarray(q[j]) for q in parts]) for j in range(4)]
@@ -73,7 +77,18 @@ def test_tile_rows(case, rows):
     t, harm, _, _ = _tile(p, 0)
     n0 = max(512, math.ceil(64 * 64 * rows / harm))
     om = _batch(p, n0 + 3, (rows - 1e-3) * t * KPAR)
-    _compare(p, om)
+    _compare(p, om, 1)
+
+
+@pytest.mark.parametrize("kpar,nr", [(0.9, 9), (0.95, 10)])
+def test_most_harmonics(kpar, nr):
+    """nr = 9 resonant harmonics, the most that tables hold (and the build's
+    largest LDS), and one past it"""
+    p = cases.kappa_case()
+    t, _, lo, up = _tile(p, 0, kpar)
+    om = _batch(p, 4000, 1.9 * t * kpar)
+    assert math.ceil(np.max(om.real) + kpar * max(abs(lo), abs(up))) + 1 == nr
+    _compare(p, om, 1 if nr <= 9 else 0, kpar)
 
 
 @pytest.mark.parametrize("form", ["at", "below", "deep", "no_norm", "nan"])
@@ -92,4 +107,4 @@ def test_rule_edges(form):
     # resonances at the ends of the accepted momenta
     om[7] = KPAR * lo + 0.5j * om[1].imag
     om[12] = KPAR * up * (1 - 1e-15) + 0.5j * om[1].imag
-    _compare(p, om)
+    _compare(p, om, 0 if form in ("below", "deep") else 1)
