@@ -547,13 +547,15 @@ OmBounds bounds_of(const double *om, int n) {
 // about twice its evaluations, so the tables are built from 64 row sums per tile
 // on.  A Chebyshev continuation's row sums cost a third of a kappa fit's, and most
 // of its tiles are clipped (96 x 64 omegas: 99 us of row sums, 250 us of tables),
-// so it keeps them.
+// so it keeps them.  The tiles lie at Im p = m Im om / kpar <= 0: with kpar < 0 that
+// is a growing omega, which has no Landau term, and every row would be left to the
+// row sums.
 constexpr int LAND_MIN = 512;
 
 int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, int RB, LandTabs &T, bool &use) {
   use = false;
   if (n < LAND_MIN || (h->lgen & 2) == 0 || !(b.re_lo <= b.re_hi) || !std::isfinite(b.re_lo) ||
-      !std::isfinite(b.re_hi) || !std::isfinite(b.im_lo) || b.im_lo > 0.0)
+      !std::isfinite(b.re_hi) || !std::isfinite(b.im_lo) || b.im_lo > 0.0 || !(h->prob.kpar > 0.0))
     return ALPSG_OK;
   const double kpar = h->prob.kpar;
   std::memset(&T, 0, sizeof(T));
@@ -568,14 +570,14 @@ int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, int RB, LandTabs &T, b
     // (a little wider: an edge momentum may round past the last tile; few bits, so
     // the centres' imaginary parts are exact)
     const double t = (double)(float)((U - L) * (1.0 + 1e-6) / LT_NX);
-    const double depth = -h->ms[s] * b.im_lo / std::fabs(kpar);
+    const double depth = -h->ms[s] * b.im_lo / kpar;
     const double ny = std::floor(depth / t) + 1.0;
     // a resonance needs m Re om - kpar p = n q within the grid
     const double q = std::fabs(h->qs[s]);
     const double e = std::max(std::fabs(h->ms[s] * b.re_lo), std::fabs(h->ms[s] * b.re_hi)) +
-                     std::fabs(kpar) * std::max(std::fabs(L), std::fabs(U));
+                     kpar * std::max(std::fabs(L), std::fabs(U));
     const int nr = (int)std::min((double)S.nmax, std::ceil(e / q) + 1.0);
-    const double rows = std::fabs(kpar) * (U - L) / q;  // resonant harmonics of an omega
+    const double rows = kpar * (U - L) / q;  // resonant harmonics of an omega
     if (!(t > 0.0) || !(ny <= LT_NY) || nr > LT_NR || (double)n * rows < 64.0 * LT_NX * ny) continue;
     LandTab &tb = T.sp[s];
     tb.ny = (int)ny;

@@ -91,6 +91,14 @@ def test_most_harmonics(kpar, nr):
     _compare(p, om, 1 if nr <= 9 else 0, kpar)
 
 
+def test_negative_kpar():
+    """Im p = m Im om / kpar is positive for damped omegas: no tile covers it, and
+    none is built"""
+    p = cases.kappa_case()
+    t, _, _, _ = _tile(p, 0)
+    _compare(p, _batch(p, 1600, 1.9 * t * KPAR), 0, -KPAR)
+
+
 @pytest.mark.parametrize("form", ["at", "below", "deep", "no_norm", "nan"])
 def test_rule_edges(form):
     p = cases.kappa_two_fits()
