@@ -345,6 +345,7 @@ inline size_t f_pp(int nspec, int nperp, int npar, int s, int iperp, int ipar, i
 // (nch_b) and its harmonic blocks (rb).
 struct LaunchShape {
   int nch_a, w_a, rc_a, nch_b, rb;
+  int nch_l = 0;  // lanes of the row sums of kappa species beside Landau tables, 0: nch_b
 };
 
 int size_bucket(int n) {
@@ -368,7 +369,10 @@ int size_bucket(int n) {
 // blocks until the chip is full.  Device time of the three kernels with the
 // shapes before (8, 2 and 1 lanes from 2048, 8192 and 32768) and these, protons
 // and electrons on 128 x 256: 784 omegas 198 -> 141 us, 3192 537 -> 205,
-// 11990 1439 -> 330, 47961 1107 -> 693.
+// 11990 1439 -> 330, 47961 1107 -> 693.  The row sums of a kappa species beside
+// another's tables want more lanes than the ladder: the resonant kernels of a core,
+// a beam and electrons at 4, 8, 16, 32 lanes, 4500 omegas on 200 x 400: 339, 283,
+// 289, 315 us; 20000 on 200 x 400: 503, 385, 381, 432.
 LaunchShape pick_shape(int n, int rows) {
   LaunchShape s;
   if (n >= 1024) {
@@ -388,6 +392,7 @@ LaunchShape pick_shape(int n, int rows) {
     s = {64, 4, 16, 64, 8};
   }
   s.rc_a = std::max(1, std::min(s.rc_a, (rows + s.w_a - 1) / s.w_a));
+  s.nch_l = std::max(s.nch_b, 16);
   return s;
 }
 
@@ -552,7 +557,8 @@ OmBounds bounds_of(const double *om, int n) {
 // row sums.
 constexpr int LAND_MIN = 512;
 
-int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, int RB, LandTabs &T, bool &use) {
+int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, const LaunchShape &sh, LandTabs &T,
+                  bool &use) {
   use = false;
   if (n < LAND_MIN || (h->lgen & 2) == 0 || !(b.re_lo <= b.re_hi) || !std::isfinite(b.re_lo) ||
       !std::isfinite(b.re_hi) || !std::isfinite(b.im_lo) || b.im_lo > 0.0 || !(h->prob.kpar > 0.0))
@@ -590,7 +596,7 @@ int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, int RB, LandTabs &T, b
     if (h->landcut.ensure((size_t)ALPSG_MAXSPEC * LT_MAXP) != hipSuccess ||
         h->landc[s].ensure(tiles * (nr + 1) * 3 * LT_J * 4) != hipSuccess ||
         h->landok[s].ensure(tiles) != hipSuccess ||
-        h->landneed.ensure((size_t)h->nspec * RB * n) != hipSuccess) {
+        h->landneed.ensure((size_t)h->nspec * sh.rb * n) != hipSuccess) {
       (void)hipGetLastError();  // no room: the row sums need none
       continue;
     }
@@ -602,6 +608,8 @@ int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, int RB, LandTabs &T, b
     use = true;
   }
   if (!use) return ALPSG_OK;
+  for (int s = 0; s < h->nspec; ++s)
+    if (h->prob.sp[s].fit_kappa && T.sp[s].c == nullptr) T.rest = sh.nch_l ? sh.nch_l : sh.nch_b;
   T.need = h->landneed.p;
   HIPCHK(launch_land_build(h->st, h->prob_d.p, h->nspec, ny_max, nr_max, T));
   return ALPSG_OK;
@@ -612,7 +620,7 @@ int disp_device(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_de
   if (const int rc = ensure_series(h, n)) return rc;
   LandTabs tabs;
   bool use_tabs = false;
-  if (const int rc = landau_tables(h, n, ob, sh.rb, tabs, use_tabs)) return rc;
+  if (const int rc = landau_tables(h, n, ob, sh, tabs, use_tabs)) return rc;
   const int ns = h->nspec;
   const int TW = sh.w_a * sh.rc_a;
   HIPCHK(h->det_d.ensure(n));
@@ -772,7 +780,7 @@ int autotune(alpsg_ctx *h, int n, const double2 *om_host, int *shape_out) {
       HIPCHK(h->chiB_d.ensure((size_t)n * ns * 2 * rb * 6));
       LandTabs tabs;
       bool ut = false;
-      if (const int rc = landau_tables(h, n, ob, rb, tabs, ut)) return rc;
+      if (const int rc = landau_tables(h, n, ob, LaunchShape{0, 0, 0, nb, rb}, tabs, ut)) return rc;
       float t;
       int rc_ = time_launch(
           [&]() {
@@ -2400,7 +2408,7 @@ int alpsg_landau_work(alpsg_handle h, int n, const double *om, double *work2) {
   const LaunchShape sh = shape_for(h, n);
   LandTabs tabs;
   bool use = false;
-  if (const int rc = landau_tables(h, n, bounds_of(om, n), sh.rb, tabs, use)) return rc;
+  if (const int rc = landau_tables(h, n, bounds_of(om, n), sh, tabs, use)) return rc;
   if (!use) return ALPSG_OK;
   HIPCHK(h->om_d.ensure(n));
   HIPCHK(h->chiB_d.ensure((size_t)n * h->nspec * 2 * sh.rb * 6));

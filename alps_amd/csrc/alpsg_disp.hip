@@ -1776,6 +1776,10 @@ __global__ __launch_bounds__(64) void k_resonant_gen(const ProbDev *__restrict__
                         blockIdx.x, blockIdx.y, threadIdx.x, win_dyn, pvw);
 }
 
+// the rows of a k_resonant_kappa launch: every species' (no tables), those that the
+// tables left, those of the species without tables
+enum KappaRows { KR_ALL, KR_LEFT, KR_REST };
+
 // The Landau part of the kappa species (part 3): the lean power leaves the
 // pass short of four wavefronts per SIMD; three, with a few spills outside
 // the evaluation loop, run it 12 % faster than the two of its natural
@@ -1784,10 +1788,11 @@ template <int NCH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_resonant_kappa(
     const ProbDev *__restrict__ probp, int nom, const double2 *__restrict__ om_in,
     const int *__restrict__ active, double2 *__restrict__ chiB, double2 *__restrict__ lowB,
-    const int *__restrict__ pidx, bool use_tabs, LandTabs tabs) {
+    const int *__restrict__ pidx, KappaRows which, LandTabs tabs) {
+  if (which != KR_ALL && (tabs.sp[blockIdx.y].c != nullptr) != (which == KR_LEFT)) return;
   resonant_body<NCH, 3>(probp, nom, om_in, active, chiB, lowB, pidx, gridDim.z, blockIdx.z,
                         blockIdx.x, blockIdx.y, threadIdx.x, nullptr, PV_WIN,
-                        use_tabs ? tabs.sp[blockIdx.y] : LandTab{}, tabs.need);
+                        which == KR_LEFT ? tabs.sp[blockIdx.y] : LandTab{}, tabs.need);
 }
 
 // The principal-value and Landau parts in one launch (small batches, where a
@@ -2069,9 +2074,6 @@ hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob,
   if (pidx != nullptr && (nch != 64 || tabs != nullptr)) return hipErrorInvalidValue;
   const LandTabs tb = tabs != nullptr ? *tabs : LandTabs{};
   const bool ut = tabs != nullptr;
-  // (the rows left to the row sums are few: many lanes each, and a wavefront
-  // without any ends at once)
-  const int nchl = !ut ? nch : (nom <= 16384 ? 64 : 16);
   if (ut)
     hipLaunchKernelGGL(k_resonant_tab, dim3((nom + 15) / 16, nspec, RB), dim3(64), 0, st, prob, nom,
                        om, active, chiB, lowB, tb);
@@ -2094,11 +2096,17 @@ hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob,
 #undef RS
   if (!done) return hipErrorInvalidValue;
 #define RL(N)                                                                                  \
-  if (nchl == N)                                                                               \
+  if (lanes == N)                                                                              \
     hipLaunchKernelGGL((k_resonant_kappa<N>), dim3((nom + (64 / N) - 1) / (64 / N), nspec, RB), \
-                       dim3(64), 0, st, prob, nom, om, active, chiB, lowB, pidx, ut, tb);
-  if (lgen & 2) {
-    RL(4) RL(8) RL(16) RL(32) RL(64)
+                       dim3(64), 0, st, prob, nom, om, active, chiB, lowB, pidx, which, tb);
+  auto kappa = [&](int lanes, KappaRows which) { RL(4) RL(8) RL(16) RL(32) RL(64) };
+  if (!ut) {
+    if (lgen & 2) kappa(nch, KR_ALL);
+  } else {
+    // the rows that the tables left are few: many lanes each, and a wavefront without
+    // any ends at once; a species without tables has all of its rows
+    kappa(nom <= 16384 ? 64 : 16, KR_LEFT);
+    if (tb.rest) kappa(tb.rest, KR_REST);
   }
 #undef RL
   return hipGetLastError();

@@ -99,6 +99,26 @@ def test_negative_kpar():
     _compare(p, _batch(p, 1600, 1.9 * t * KPAR), 0, -KPAR)
 
 
+@pytest.mark.parametrize("shape", [(8, 4, 4, 8, 2), (1, 4, 4, 4, 1)])
+def test_species_without_tables_keep_their_lanes(shape):
+    """The electrons' one resonant harmonic is not worth tables: their row sums take
+    the shape's lanes, with the protons' tables (800 omegas) and without any (400),
+    so their chi is the same to the last bit"""
+    from alps_amd.engine import Engine
+    p = cases.kappa_case()
+    t, _, _, _ = _tile(p, 0)
+    om = _batch(p, 800, 0.99 * t * KPAR)
+    E = Engine(p)
+    E.set_k(KPERP, KPAR)
+    E.set_sweep_series(False)
+    for n in (800, 400):
+        E.set_shape(n, shape)
+    assert E.landau_work(om)[0] == 1 and E.landau_work(om[:400])[0] == 0
+    chi = [np.asarray(E.disp_batch(om[:n], want_tensors=True)[1])[:384, 1] for n in (800, 400)]
+    E.close()
+    assert np.array_equal(*chi)
+
+
 @pytest.mark.parametrize("form", ["at", "below", "deep", "no_norm", "nan"])
 def test_rule_edges(form):
     p = cases.kappa_two_fits()
