@@ -2103,9 +2103,11 @@ hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob,
   if (!ut) {
     if (lgen & 2) kappa(nch, KR_ALL);
   } else {
-    // the rows that the tables left are few: many lanes each, and a wavefront without
-    // any ends at once; a species without tables has all of its rows
-    kappa(nom <= 16384 ? 64 : 16, KR_LEFT);
+    // the rows that the tables left are few, and a wavefront without any ends at once:
+    // 16 lanes each (64, 16, 8 lanes of 16384 omegas with none left: the resonant
+    // kernels 345, 310, 303 us; of 16000 with a sixth left 300, 259, 262; of 5400 with
+    // 155 left 152, 155, 166); a species without tables has all of its rows
+    kappa(16, KR_LEFT);
     if (tb.rest) kappa(tb.rest, KR_REST);
   }
 #undef RL
