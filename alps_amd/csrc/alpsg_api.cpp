@@ -410,7 +410,10 @@ LaunchShape shape_for(const alpsg_ctx *h, int n) {
 }
 
 // the small-batch sweep (k_sweep_req<REQ_NCH, REQ_W, REQ_K> over REQ_TW / REQ_W
-// workgroups per omega) for batches of at most REQ_MAX_N omegas
+// workgroups per omega) for batches of at most REQ_MAX_N omegas.  det D of such a
+// batch is one launch whatever its size and Landau forms, against three in a captured
+// graph (whole call, 1 and 16 omegas on 64 x 128: Maxwellian species 52, 54 -> 33, 39
+// us; kappa 54, 72 -> 35, 51; Chebyshev 62, 71 -> 42, 53)
 constexpr int REQ_MAX_N = 16, REQ_NCH = 32, REQ_W = 4, REQ_TW = 64, REQ_K = 4;
 constexpr int PIN_MAX = 4096;  // batches up to this size copy om and det through pinned memory
 
@@ -1009,7 +1012,8 @@ int osc_graph_batch(alpsg_ctx *h, const alpsg_root_params *rp, int n, cplx *om, 
     hipError_t e = hipSuccess;
     for (int k = 0; k < OSC_K && e == hipSuccess; ++k) {
       if (req && REQ_W == 4 && REQ_NCH == 32 && REQ_K == 4) {
-        // the whole round in one launch
+        // the whole round in one launch (two where a species takes the general
+        // Landau form)
         e = launch_small(h->st, sh.nch_b, sh.rb, REQ_TW / REQ_W, h->prob_d.p, ns, n, h->om_d.p,
                          h->chiA_d.p, h->chiB_d.p, h->det_d.p, h->zidx.p, h->lgen, h->done_d.p,
                          h->osc_d.p, h->oscctl_d.p);

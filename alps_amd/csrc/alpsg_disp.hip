@@ -2324,31 +2324,16 @@ __global__ __launch_bounds__(256) void k_assemble_osc(
   assemble_osc(probp, nom, W, RB, om_in, chiA, chiB, det, nspec, S, om_next, round_ctr, remaining);
 }
 
-// A small batch in one launch.  Workgroups [0, nom RC) run the request sweep
-// (omega b % nom, workgroup b / nom of RC; 32 lanes per row pair, 4 records in
-// flight), the others four resonant wavefronts each (every part and harmonic
-// block).  The workgroup that finishes last assembles det D of every omega and,
-// with OSC, feeds it to the solves: a launch of its own for that costs its
-// start and end, and every one of them writes back and refills what it shares
-// with the next.  Each workgroup's partial sums are released to the device
-// before it counts itself in done; the last one acquires them, and sets done
-// back to zero for the next launch (a secant round of one root, two species of
-// 50 x 100: 11.1 + 6.2 us and the gap between two launches, 15.1 us so).
-// om and det may lie in host memory that the device can reach.  Held to two
-// wavefronts per SIMD: 16 omegas of three species are two workgroups a CU (their
-// rounds 57 us at one, 49 at two).
-constexpr int SMALL_STAGE = 1024;
-template <int NCHR, int GEN, bool OSC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_small(const ProbDev *__restrict__ probp, int nom,
-                                               double2 *om, double2 *chiA, double2 *chiB,
-                                               const int *__restrict__ zidx, int RC, int RB,
-                                               int nspec, double2 *det, int *done,
-                                               alpsg_osc::OscMachine *S, int *ctl) {
+// The request sweep and both resonant parts of a small batch: workgroups
+// [0, nom RC) run the sweep (omega b % nom, workgroup b / nom of RC; 32 lanes per
+// row pair, 4 records in flight), the others four resonant wavefronts each (every
+// part and harmonic block)
+template <int NCHR, int GEN>
+__device__ __forceinline__ void small_sums(const ProbDev *__restrict__ probp, int nom,
+                                           const double2 *om, double2 *chiA, double2 *chiB,
+                                           const int *__restrict__ zidx, int RC, int RB, int nspec) {
   constexpr int OMB = 64 / NCHR;
   __shared__ double win[4][OMB * 2 * PV_WIN];
-  __shared__ int last;
-  if constexpr (OSC)
-    if (ctl[1] == 0) return;  // every solve has finished: nothing to evaluate
   const int A = nom * RC;
   const int b = blockIdx.x;
   const int gx = (nom + OMB - 1) / OMB;
@@ -2372,6 +2357,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                                lane, win[wave]);
     }
   }
+}
+
+// The sums alone, for the secant rounds of a plasma with the general Landau form
+// (k_assemble_osc follows): their evaluation of the fit is a call, and the assembly in
+// the same kernel costs it registers.  A solve of 4 and of 16 roots on 64 x 128, whole
+// call, with one launch a round and with two: Chebyshev species 775 and 946 us, 717
+// and 871; a kappa species beside it 403 and 493, 365 and 472.
+template <int NCHR, int GEN>
+__global__ __launch_bounds__(256) void k_small_sums(const ProbDev *__restrict__ probp, int nom,
+                                                    const double2 *__restrict__ om, double2 *chiA,
+                                                    double2 *chiB, const int *__restrict__ zidx,
+                                                    int RC, int RB, int nspec,
+                                                    const int *__restrict__ remaining) {
+  if (*remaining == 0) return;  // every solve has finished: nothing to evaluate
+  small_sums<NCHR, GEN>(probp, nom, om, chiA, chiB, zidx, RC, RB, nspec);
+}
+
+// A small batch in one launch: small_sums, then the workgroup that finishes last
+// assembles det D of every omega and, with OSC, feeds it to the solves: a launch of
+// its own for that costs its start and end, and every one of them writes back and
+// refills what it shares with the next.  Each workgroup's partial sums are released
+// to the device before it counts itself in done; the last one acquires them, and sets
+// done back to zero for the next launch.  A secant round of one root, two species of
+// 50 x 100: 11.1 + 6.2 us and the gap between two launches, 15.1 us so; a solve of 1,
+// 4 and 16 roots, whole call: protons and electrons on 64 x 128 341, 394, 482 us with
+// two launches a round, 304, 380, 451 so; three kappa species on 128 x 256 411, 419,
+// 590 and 375, 393, 565.
+// om and det may lie in host memory that the device can reach.  Held to two
+// wavefronts per SIMD: 16 omegas of three species are two workgroups a CU (their
+// rounds 57 us at one, 49 at two).
+constexpr int SMALL_STAGE = 1024;
+template <int NCHR, int GEN, bool OSC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_small(const ProbDev *__restrict__ probp, int nom,
+                                               double2 *om, double2 *chiA, double2 *chiB,
+                                               const int *__restrict__ zidx, int RC, int RB,
+                                               int nspec, double2 *det, int *done,
+                                               alpsg_osc::OscMachine *S, int *ctl) {
+  __shared__ int last;
+  if constexpr (OSC)
+    if (ctl[1] == 0) return;  // every solve has finished: nothing to evaluate
+  small_sums<NCHR, GEN>(probp, nom, om, chiA, chiB, zidx, RC, RB, nspec);
   // every wavefront's stores are acknowledged, then one lane releases them all
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
@@ -2424,10 +2450,18 @@ hipError_t launch_small(hipStream_t st, int nchr, int RB, int RC, const ProbDev 
   if (nom > 256 || 6 * nspec > 256 || lgen < 0 || lgen > 3) return hipErrorInvalidValue;
 #define RDG(N, G)                                                                                  \
   if (lgen == G) {                                                                                 \
-    if (S != nullptr)                                                                              \
+    if constexpr ((G & 1) != 0) {                                                                  \
+      if (S != nullptr) {                                                                          \
+        hipLaunchKernelGGL((k_small_sums<N, G>), dim3(grid), dim3(256), 0, st, prob, nom, om,      \
+                           chiA, chiB, zidx, RC, RB, nspec, ctl + 1);                              \
+        hipLaunchKernelGGL(k_assemble_osc, dim3(1), dim3(256), 0, st, prob, nom, RC, RB, om, chiA, \
+                           chiB, det, nspec, S, om, ctl, ctl + 1);                                 \
+      }                                                                                            \
+    } else if (S != nullptr) {                                                                     \
       hipLaunchKernelGGL((k_small<N, G, true>), dim3(grid), dim3(256), 0, st, prob, nom, om, chiA, \
                          chiB, zidx, RC, RB, nspec, det, done, S, ctl);                            \
-    else                                                                                           \
+    }                                                                                              \
+    if (S == nullptr)                                                                              \
       hipLaunchKernelGGL((k_small<N, G, false>), dim3(grid), dim3(256), 0, st, prob, nom, om,      \
                          chiA, chiB, zidx, RC, RB, nspec, det, done, S, ctl);                      \
   }

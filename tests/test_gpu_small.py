@@ -46,3 +46,22 @@ def test_roots_in_turn():
         om, _, _ = E.secant_osc_batch(root * (1.0 + 1e-3 * np.exp(1j * np.arange(n))))
         assert np.all(np.abs(om - root) <= p.roots.D_prec), n
     E.close()
+
+
+@pytest.mark.parametrize("case", ["kappa_case", "poly_case", "kappa_poly_mix"])
+def test_roots_of_every_landau_form(case):
+    """secant rounds of one launch (kappa fits alone) and of two (a species with the
+    general Landau form) against the solves stepped on the host: the same steps to
+    rounding, so well within the D_prec that ends them"""
+    from alps_amd.engine import Engine
+    p = getattr(cases, case)()
+    E = Engine(p)
+    E.set_k(0.3, 0.4)
+    for n in (1, 3, 16, 2, 17, 1):
+        g = 0.4 - 0.01j + 2e-3 * np.exp(1j * np.arange(n))
+        om, _, it = E.secant_osc_batch(g)
+        E.set_plain_roots(True)
+        ref, _, it_ref = E.secant_osc_batch(g)
+        E.set_plain_roots(False)
+        assert np.array_equal(it, it_ref) and np.all(np.abs(om - ref) <= p.roots.D_prec), n
+    E.close()
