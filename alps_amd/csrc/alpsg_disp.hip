@@ -1331,8 +1331,9 @@ enum { LM_GEN = 0, LM_UNI = 1, LM_KAPPA = 2 };
 // Landau sums L_a = sum_iperp h a(n,iperp) K(iperp) of this lane, and the
 // early-return flag of landau_integrate.  When every fit of the species is a
 // Maxwellian whose ppar parameters do not depend on pperp, exp(-u2 (p-u3)^2) is
-// the same for every iperp and is evaluated once (bit-identical values).
-template <int NCH, int LM>
+// the same for every iperp and is evaluated once (bit-identical values).  PRE: the
+// last tested row first.
+template <int NCH, int LM, bool PRE>
 __device__ void landau_part(const SpecDev &S, const ProbDev &Pd, int an, const RowClass &rc,
                             double omr, double omi, int c, cd L[3], int &zero) {
   const double *__restrict__ arow = S.atab + (size_t)an * (S.nperp + 1) * ATAB_STRIDE;
@@ -1396,12 +1397,14 @@ __device__ void landau_part(const SpecDev &S, const ProbDev &Pd, int an, const R
     // pperp, where f0 is smallest, is the one that underflows or is clipped first:
     // its three values come first, a lane each, and a zero ends the term there
     // (a 96 x 64 map of a Chebyshev continuation: 331 us of these sums, 236 so)
-    static_assert(NCH >= 3, "a lane for each value of the last tested row");
-    cd last = mk(1.0, 0.0);
-    if (c < 3) last = F(c == 2 ? nperp : nperp - 1, c == 0 ? 1 : (c == 1 ? -1 : 0));
-    if (gor<NCH>(czero(last) ? 1 : 0)) {
-      zero = 1;
-      return;
+    if constexpr (PRE) {
+      static_assert(NCH >= 3, "a lane for each value of the last tested row");
+      cd last = mk(1.0, 0.0);
+      if (c < 3) last = F(c == 2 ? nperp : nperp - 1, c == 0 ? 1 : (c == 1 ? -1 : 0));
+      if (gor<NCH>(czero(last) ? 1 : 0)) {
+        zero = 1;
+        return;
+      }
     }
     const int blk = (nperp + 1 + NCH - 1) / NCH;
     const int r0 = c * blk, r1 = min(r0 + blk, nperp + 1) - 1;
@@ -1541,8 +1544,12 @@ __device__ __forceinline__ int land_tile(const LandTab &T, int an, double pr, do
 // other species.  PV writes partial slots rb, the Landau launches slots RB + rb
 // of chiB / lowB (each species by exactly one of PART 1, 2, 3).
 // One wavefront's share of k_resonant: omega block bx, species by, harmonic
-// block rb of RB; win_lds holds (64 / NCH) windows of 2 pvw doubles.
-template <int NCH, int PART>
+// block rb of RB; win_lds holds (64 / NCH) windows of 2 pvw doubles.  PRE (the
+// general Landau form): the last tested row first.  Not in the kernels of small
+// batches, whose lanes have a row or two each: the row's evaluation comes on top of
+// their six to eight (a solve of a Chebyshev species on 64 x 128: 700 us, 660
+// without), nor for kappa fits, which fall off as a power and are never zero.
+template <int NCH, int PART, bool PRE = (PART == 2)>
 __device__ __forceinline__ void resonant_body(const ProbDev *__restrict__ probp, int nom,
                                               const double2 *__restrict__ om_in,
                                               const int *__restrict__ active,
@@ -1634,7 +1641,7 @@ __device__ __forceinline__ void resonant_body(const ProbDev *__restrict__ probp,
     if constexpr (PART != 0) {
       cd L[3] = {mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0)};
       int zero = 0;
-      landau_part<NCH, PART == 1 ? LM_UNI : (PART == 3 ? LM_KAPPA : LM_GEN)>(S, Pd, an, rc, omr,
+      landau_part<NCH, PART == 1 ? LM_UNI : (PART == 3 ? LM_KAPPA : LM_GEN), PRE>(S, Pd, an, rc, omr,
                                                                              omi, c, L, zero);
       zero = gor<NCH>(zero);
       if (!zero) {
@@ -1814,8 +1821,8 @@ __global__ __launch_bounds__(64) void k_resonant_all(const ProbDev *__restrict__
   resonant_body<NCH, 1>(probp, nom, om_in, nullptr, chiB, nullptr, pidx, RB, z - RB, bx, by, lane,
                         win);
   if constexpr ((GEN & 1) != 0)
-    resonant_body<NCH, 2>(probp, nom, om_in, nullptr, chiB, nullptr, pidx, RB, z - RB, bx, by,
-                          lane, win);
+    resonant_body<NCH, 2, false>(probp, nom, om_in, nullptr, chiB, nullptr, pidx, RB, z - RB, bx,
+                                 by, lane, win);
   if constexpr ((GEN & 2) != 0)
     resonant_body<NCH, 3>(probp, nom, om_in, nullptr, chiB, nullptr, pidx, RB, z - RB, bx, by,
                           lane, win);
@@ -2350,8 +2357,8 @@ __device__ __forceinline__ void small_sums(const ProbDev *__restrict__ probp, in
       resonant_body<NCHR, 1>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y,
                              lane, win[wave]);
       if constexpr ((GEN & 1) != 0)
-        resonant_body<NCHR, 2>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y,
-                               lane, win[wave]);
+        resonant_body<NCHR, 2, false>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB,
+                                      x, y, lane, win[wave]);
       if constexpr ((GEN & 2) != 0)
         resonant_body<NCHR, 3>(probp, nom, om, nullptr, chiB, nullptr, nullptr, RB, z - RB, x, y,
                                lane, win[wave]);
