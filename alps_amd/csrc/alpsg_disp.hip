@@ -1545,11 +1545,11 @@ __device__ __forceinline__ int land_tile(const LandTab &T, int an, double pr, do
 // of chiB / lowB (each species by exactly one of PART 1, 2, 3).
 // One wavefront's share of k_resonant: omega block bx, species by, harmonic
 // block rb of RB; win_lds holds (64 / NCH) windows of 2 pvw doubles.  PRE (the
-// general Landau form): the last tested row first.  Not in the kernels of small
-// batches, whose lanes have a row or two each: the row's evaluation comes on top of
+// general Landau form): the last tested row first.  Not with 64 lanes or in the
+// kernels of small batches, whose lanes have a row or two each: the row's evaluation comes on top of
 // their six to eight (a solve of a Chebyshev species on 64 x 128: 700 us, 660
 // without), nor for kappa fits, which fall off as a power and are never zero.
-template <int NCH, int PART, bool PRE = (PART == 2)>
+template <int NCH, int PART, bool PRE = (PART == 2 && NCH < 64)>
 __device__ __forceinline__ void resonant_body(const ProbDev *__restrict__ probp, int nom,
                                               const double2 *__restrict__ om_in,
                                               const int *__restrict__ active,
