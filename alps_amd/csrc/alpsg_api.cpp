@@ -47,7 +47,7 @@ hipError_t launch_sweep_req(hipStream_t st, int nch, int W, int RC, int K, const
 hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec, int nom,
                            const double2 *om, const int *active, double2 *chiB, double2 *lowB,
                            int lgen, const int *pidx = nullptr, int P = 0,
-                           const LandTabs *tabs = nullptr);
+                           const LandTabs *tabs = nullptr, int nch_g = 0, int nch_k = 0);
 hipError_t launch_nhds(hipStream_t st, const ProbDev *prob, int nspec, int nom, const double2 *om,
                        const int *active, double2 *chiA, double2 *lowA, const int *pidx = nullptr);
 int nhds_tables(double z, int bm_nmax, double bessel_zero, std::vector<double2> &tab);
@@ -345,7 +345,8 @@ inline size_t f_pp(int nspec, int nperp, int npar, int s, int iperp, int ipar, i
 // (nch_b) and its harmonic blocks (rb).
 struct LaunchShape {
   int nch_a, w_a, rc_a, nch_b, rb;
-  int nch_l = 0;  // lanes of the row sums of kappa species beside Landau tables, 0: nch_b
+  // lanes per omega of the Landau row sums: general form, kappa fits (0: nch_b)
+  int nch_g = 0, nch_k = 0;
 };
 
 int size_bucket(int n) {
@@ -369,10 +370,14 @@ int size_bucket(int n) {
 // blocks until the chip is full.  Device time of the three kernels with the
 // shapes before (8, 2 and 1 lanes from 2048, 8192 and 32768) and these, protons
 // and electrons on 128 x 256: 784 omegas 198 -> 141 us, 3192 537 -> 205,
-// 11990 1439 -> 330, 47961 1107 -> 693.  The row sums of a kappa species beside
-// another's tables want more lanes than the ladder: the resonant kernels of a core,
-// a beam and electrons at 4, 8, 16, 32 lanes, 4500 omegas on 200 x 400: 339, 283,
-// 289, 315 us; 20000 on 200 x 400: 503, 385, 381, 432.
+// 11990 1439 -> 330, 47961 1107 -> 693.  The Landau
+// row sums, evaluations of a fit on every pperp row, want more lanes than the ladder
+// until the wavefronts are many.  Resonant kernels at 4, 8, 16, 32 lanes, Chebyshev
+// species on 48 x 96 and 128 x 256: 255 omegas 116, 86, 67, 61 us and 236, 148, 103,
+// 81; 1024 218, 151, 120, 118 and 260, 170, 128, 145; 3000 252, 191, 183, 199 and 298,
+// 311, 283, 302; 8192 369, 308, 344, 397 and 525, 558, 587, 670.  Kappa species (the
+// rows without tables): 255 143, 96, 73, 70 on 128 x 256; 2048 288, 216, 196, 213;
+// 8192 234, 187, 193, 196.
 LaunchShape pick_shape(int n, int rows) {
   LaunchShape s;
   if (n >= 1024) {
@@ -392,7 +397,11 @@ LaunchShape pick_shape(int n, int rows) {
     s = {64, 4, 16, 64, 8};
   }
   s.rc_a = std::max(1, std::min(s.rc_a, (rows + s.w_a - 1) / s.w_a));
-  s.nch_l = std::max(s.nch_b, 16);
+  s.nch_g = s.nch_k = n < 32 ? 64 : (n < 512 ? 32 : 16);
+  if (n >= 3072) {
+    s.nch_g = s.nch_b;
+    s.nch_k = 8;
+  }
   return s;
 }
 
@@ -481,7 +490,8 @@ int disp_chain(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_dev
                                h->lgen));
   else
     HIPCHK(launch_resonant(h->st, sh.nch_b, sh.rb, h->prob_d.p, ns, n, om_dev, active_dev, B.chiB,
-                           want_low ? B.lowB : nullptr, h->lgen, nullptr, h->P, tabs));
+                           want_low ? B.lowB : nullptr, h->lgen, nullptr, h->P, tabs, sh.nch_g,
+                           sh.nch_k));
   if (h->any_bm)
     HIPCHK(launch_nhds(h->st, h->prob_d.p, ns, n, om_dev, active_dev, B.chiA,
                        want_low ? B.lowA : nullptr));
@@ -560,8 +570,7 @@ OmBounds bounds_of(const double *om, int n) {
 // row sums.
 constexpr int LAND_MIN = 512;
 
-int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, const LaunchShape &sh, LandTabs &T,
-                  bool &use) {
+int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, int RB, LandTabs &T, bool &use) {
   use = false;
   if (n < LAND_MIN || (h->lgen & 2) == 0 || !(b.re_lo <= b.re_hi) || !std::isfinite(b.re_lo) ||
       !std::isfinite(b.re_hi) || !std::isfinite(b.im_lo) || b.im_lo > 0.0 || !(h->prob.kpar > 0.0))
@@ -599,7 +608,7 @@ int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, const LaunchShape &sh,
     if (h->landcut.ensure((size_t)ALPSG_MAXSPEC * LT_MAXP) != hipSuccess ||
         h->landc[s].ensure(tiles * (nr + 1) * 3 * LT_J * 4) != hipSuccess ||
         h->landok[s].ensure(tiles) != hipSuccess ||
-        h->landneed.ensure((size_t)h->nspec * sh.rb * n) != hipSuccess) {
+        h->landneed.ensure((size_t)h->nspec * RB * n) != hipSuccess) {
       (void)hipGetLastError();  // no room: the row sums need none
       continue;
     }
@@ -612,7 +621,7 @@ int landau_tables(alpsg_ctx *h, int n, const OmBounds &b, const LaunchShape &sh,
   }
   if (!use) return ALPSG_OK;
   for (int s = 0; s < h->nspec; ++s)
-    if (h->prob.sp[s].fit_kappa && T.sp[s].c == nullptr) T.rest = sh.nch_l ? sh.nch_l : sh.nch_b;
+    if (h->prob.sp[s].fit_kappa && T.sp[s].c == nullptr) T.rest = true;
   T.need = h->landneed.p;
   HIPCHK(launch_land_build(h->st, h->prob_d.p, h->nspec, ny_max, nr_max, T));
   return ALPSG_OK;
@@ -623,7 +632,7 @@ int disp_device(alpsg_ctx *h, int n, const double2 *om_dev, const int *active_de
   if (const int rc = ensure_series(h, n)) return rc;
   LandTabs tabs;
   bool use_tabs = false;
-  if (const int rc = landau_tables(h, n, ob, sh, tabs, use_tabs)) return rc;
+  if (const int rc = landau_tables(h, n, ob, sh.rb, tabs, use_tabs)) return rc;
   const int ns = h->nspec;
   const int TW = sh.w_a * sh.rc_a;
   HIPCHK(h->det_d.ensure(n));
@@ -783,7 +792,7 @@ int autotune(alpsg_ctx *h, int n, const double2 *om_host, int *shape_out) {
       HIPCHK(h->chiB_d.ensure((size_t)n * ns * 2 * rb * 6));
       LandTabs tabs;
       bool ut = false;
-      if (const int rc = landau_tables(h, n, ob, LaunchShape{0, 0, 0, nb, rb}, tabs, ut)) return rc;
+      if (const int rc = landau_tables(h, n, ob, rb, tabs, ut)) return rc;
       float t;
       int rc_ = time_launch(
           [&]() {
@@ -1039,7 +1048,8 @@ int osc_graph_batch(alpsg_ctx *h, const alpsg_root_params *rp, int n, cplx *om, 
       }
       if (e == hipSuccess)
         e = launch_resonant(h->st, sh.nch_b, sh.rb, h->prob_d.p, ns, n, h->om_d.p, nullptr,
-                            h->chiB_d.p, nullptr, h->lgen, nullptr, h->P);
+                            h->chiB_d.p, nullptr, h->lgen, nullptr, h->P, nullptr, sh.nch_g,
+                            sh.nch_k);
       if (e == hipSuccess)
         e = launch_assemble(h->st, h->prob_d.p, ns, n, TW, sh.rb, h->om_d.p, nullptr, h->chiA_d.p,
                             h->chiB_d.p, nullptr, nullptr, nullptr, 0, nullptr, 0, h->det_d.p, nullptr,
@@ -2412,13 +2422,13 @@ int alpsg_landau_work(alpsg_handle h, int n, const double *om, double *work2) {
   const LaunchShape sh = shape_for(h, n);
   LandTabs tabs;
   bool use = false;
-  if (const int rc = landau_tables(h, n, bounds_of(om, n), sh, tabs, use)) return rc;
+  if (const int rc = landau_tables(h, n, bounds_of(om, n), sh.rb, tabs, use)) return rc;
   if (!use) return ALPSG_OK;
   HIPCHK(h->om_d.ensure(n));
   HIPCHK(h->chiB_d.ensure((size_t)n * h->nspec * 2 * sh.rb * 6));
   HIPCHK(hipMemcpyAsync(h->om_d.p, om, sizeof(double2) * n, hipMemcpyHostToDevice, h->st));
   HIPCHK(launch_resonant(h->st, sh.nch_b, sh.rb, h->prob_d.p, h->nspec, n, h->om_d.p, nullptr,
-                         h->chiB_d.p, nullptr, h->lgen, nullptr, h->P, &tabs));
+                         h->chiB_d.p, nullptr, h->lgen, nullptr, h->P, &tabs, sh.nch_g, sh.nch_k));
   const size_t per = (size_t)sh.rb * n;  // (species, harmonic block, omega)
   std::vector<unsigned char> need((size_t)h->nspec * per);
   HIPCHK(hipMemcpyAsync(need.data(), h->landneed.p, need.size(), hipMemcpyDeviceToHost, h->st));

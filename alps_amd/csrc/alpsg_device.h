@@ -142,7 +142,7 @@ struct LandTabs {
   LandTab sp[ALPSG_DMAXSPEC];
   // [species][harmonic block][omega]: a row of this omega is left to the row sums
   unsigned char *need;
-  int rest;  // lanes of the row sums of the kappa species without a table, 0: none
+  bool rest;  // some kappa species has no table
 };
 
 // ---------------------------------------------------------------------------

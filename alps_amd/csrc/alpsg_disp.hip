@@ -2073,12 +2073,14 @@ hipError_t launch_sweep_req(hipStream_t st, int nch, int W, int RC, int K, const
 
 // lgen: bit 0 set if a species takes the part-2 Landau form, bit 1 if one
 // takes the part-3 (kappa) form; P: positions_principal of every problem of
-// the launch (<= 0: unknown, the largest window)
+// the launch (<= 0: unknown, the largest window); nch_g, nch_k: lanes per omega of the
+// row sums of part 2 and of part 3, 0: nch
 hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec, int nom,
                            const double2 *om, const int *active, double2 *chiB, double2 *lowB,
-                           int lgen, const int *pidx, int P, const LandTabs *tabs) {
+                           int lgen, const int *pidx, int P, const LandTabs *tabs, int nch_g,
+                           int nch_k) {
   if (nom <= 0) return hipSuccess;
-  if (pidx != nullptr && (nch != 64 || tabs != nullptr)) return hipErrorInvalidValue;
+  if (pidx != nullptr && (nch != 64 || nch_g != 0 || nch_k != 0 || tabs != nullptr)) return hipErrorInvalidValue;
   const LandTabs tb = tabs != nullptr ? *tabs : LandTabs{};
   const bool ut = tabs != nullptr;
   if (ut)
@@ -2094,28 +2096,34 @@ hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob,
                        lowB, pidx, pvw);                                                       \
     hipLaunchKernelGGL((k_resonant<N, 1>), dim3(grid, nspec, RB), dim3(64), 0, st, prob, nom,  \
                        om, active, chiB, lowB, pidx, pvw);                                     \
-    if (lgen & 1)                                                                              \
-      hipLaunchKernelGGL((k_resonant_gen<N>), dim3(grid, nspec, RB), dim3(64), 0, st, prob, nom, \
-                         om, active, chiB, lowB, pidx, pvw);                                   \
     done = true;                                                                               \
   }
   RS(4) RS(8) RS(16) RS(32) RS(64)
 #undef RS
   if (!done) return hipErrorInvalidValue;
+  const int lg = nch_g != 0 ? nch_g : nch, lk = nch_k != 0 ? nch_k : nch;
+#define RG(N)                                                                                  \
+  if (lg == N)                                                                                 \
+    hipLaunchKernelGGL((k_resonant_gen<N>), dim3((nom + (64 / N) - 1) / (64 / N), nspec, RB),  \
+                       dim3(64), 0, st, prob, nom, om, active, chiB, lowB, pidx, pvw);
+  if (lgen & 1) {
+    RG(4) RG(8) RG(16) RG(32) RG(64)
+  }
+#undef RG
 #define RL(N)                                                                                  \
   if (lanes == N)                                                                              \
     hipLaunchKernelGGL((k_resonant_kappa<N>), dim3((nom + (64 / N) - 1) / (64 / N), nspec, RB), \
                        dim3(64), 0, st, prob, nom, om, active, chiB, lowB, pidx, which, tb);
   auto kappa = [&](int lanes, KappaRows which) { RL(4) RL(8) RL(16) RL(32) RL(64) };
   if (!ut) {
-    if (lgen & 2) kappa(nch, KR_ALL);
+    if (lgen & 2) kappa(lk, KR_ALL);
   } else {
     // the rows that the tables left are few, and a wavefront without any ends at once:
     // 16 lanes each (64, 16, 8 lanes of 16384 omegas with none left: the resonant
     // kernels 345, 310, 303 us; of 16000 with a sixth left 300, 259, 262; of 5400 with
     // 155 left 152, 155, 166); a species without tables has all of its rows
     kappa(16, KR_LEFT);
-    if (tb.rest) kappa(tb.rest, KR_REST);
+    if (tb.rest) kappa(lk, KR_REST);
   }
 #undef RL
   return hipGetLastError();

@@ -75,7 +75,8 @@ hipError_t launch_sweep_req(hipStream_t st, int nch, int W, int RC, int K, const
                             bool reduce);
 hipError_t launch_resonant(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec, int nom,
                            const double2 *om, const int *active, double2 *chiB, double2 *lowB,
-                           int lgen, const int *pidx, int P, const LandTabs *tabs = nullptr);
+                           int lgen, const int *pidx, int P, const LandTabs *tabs = nullptr,
+                           int nch_g = 0, int nch_k = 0);
 hipError_t launch_resonant_all(hipStream_t st, int nch, int RB, const ProbDev *prob, int nspec,
                                int nom, const double2 *om, double2 *chiB, int lgen,
                                const int *pidx);

@@ -79,6 +79,25 @@ def test_omegas_far_off_the_grid(case, n):
     E.close()
 
 
+@pytest.mark.parametrize("case", ["poly_case", "kappa_case", "kappa_poly_mix"])
+def test_default_lanes_of_the_row_sums(case):
+    """the untuned batches on both sides of each change of the Landau row sums' lanes"""
+    p = getattr(cases, case)()
+    rng = np.random.default_rng(3)
+    oms = rng.uniform(0.05, 1.5, 5) - 0.3j * rng.uniform(0.01, 0.9, 5)
+    O, E = Oracle(p), _engine(p)
+    assert O.set_k(0.3, 0.3) == E.set_k(0.3, 0.3)
+    ref = [O.disp(om, want_tensors=True) for om in oms]
+    for n in (31, 32, 511, 512, 3071, 3072):
+        _, chi, low, _ = E.disp_batch(np.resize(oms, n), want_tensors=True)
+        for k in list(range(5)) + [n - 1]:
+            _, c, lo, _ = ref[k % 5]
+            for s in range(p.nspec):
+                for g, o in ((chi[k, s], c[s]), (low[k, s], lo[s])):
+                    assert np.max(np.abs(g - o)) <= TOL * np.max(np.abs(o)), (n, k, s)
+    E.close()
+
+
 def test_three_species():
     p = cases.three_species()
     _check(p, 0.5, 0.2, cases.BRANCH_OMEGAS)
