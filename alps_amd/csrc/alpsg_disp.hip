@@ -349,9 +349,12 @@ __device__ __forceinline__ void sweep_nodes_pf(cdptr srows, cdptr pa, int npar, 
   }
 }
 
-// the largest cancellation of G/m against C/den that the split form of a row is
-// used at: at 256 det D of the 256 x 256 map was 5e-14 from the 64-bit sums, at
-// 16 (7 % of that map's time more) it is 5e-15, as with the U r products
+// The largest cancellation of G/m against C/den that the split form of a row is
+// used at.  256 x 256 omegas of protons and electrons on 128 x 256, shape {1, 2, 4}:
+// at 256, 64, 16, 4 k_sweep takes 454, 483, 478, 588 us, and det D is 5.2e-14, 5.1e-15,
+// 5.1e-15, 5.1e-15 (norm) from the 64-bit sums; the median over points of 15 batches
+// of other sizes and plasmas is 4.4e-15, 3.7e-15, 3.3e-15, 3.1e-15, the last as with
+// the U r products throughout.
 constexpr double SPLIT_MAX = 16.0;
 constexpr int LPA = 1025;  // ppar points a sweep workgroup keeps in LDS (npar <= 1024)
 constexpr int LPA_REQ = 2056;  // the request sweep's: every species' grid at once up to this
@@ -1361,7 +1364,7 @@ __device__ void landau_part(const SpecDev &S, const ProbDev &Pd, int an, const R
   if constexpr (UNI) {
     if (S.lsum != nullptr) {
       // eval_fit = c0(iperp) E(p): the sum over iperp is two omega-independent
-      // per-k sums (k_lsum) times A = (E(p+d) - E(p-d))/2d and (om - km p) E(p);
+      // per-k sums (lsum_block) times A = (E(p+d) - E(p-d))/2d and (om - km p) E(p);
       // the zero test needs only the smallest |c0| of its rows (a product
       // c0 x rounds to zero for some row iff it does for the smallest |c0|)
       if (c == 0) {

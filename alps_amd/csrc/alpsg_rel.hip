@@ -1748,7 +1748,12 @@ __global__ __launch_bounds__(64) void k_rel_landau(
 RelSplit rel_split(int nom) {
   // A few omegas (secant steps) need the parts to fill the chip: one omega is
   // 16 x 8 + 31 x 4 workgroups at nmax 30.  A large batch fills it without, and
-  // the parts would only add partial slots to write and sum.
+  // the parts would only add partial slots to write and sum.  Whole calls with
+  // tensors at {8, 4}, {4, 2}, {1, 1}, us: 200 x 400 grid 1 omega 260, 291, 457;
+  // 64: 658, 664, 820; 96: 892, 872, 935; 192: 1448, 1475, 1509; 256: 1896, 1885,
+  // 1820; 512: 3484, 3310, 3210.  100 x 200: 1: 223, 222, 275; 64: 454, 393, 437;
+  // 192: 822, 693, 729; 256: 1011, 952, 883.  The lines lie where the larger table
+  // breaks even.
   if (nom <= 64) return {8, 4};
   if (nom <= 256) return {4, 2};
   return {1, 1};

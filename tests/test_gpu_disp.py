@@ -177,9 +177,9 @@ def test_single_omega_paths_agree():
 
 
 def test_replayed_small_batches_match_the_large_batch():
-    """Batches of up to 16 omegas (det only) replay a captured graph of their
-    disp chain: every replay, interleaved with large eager batches and with a
-    change of k, equals the large-batch evaluation of the same omegas."""
+    """Batches of up to 16 omegas (det only) are one launch whose last workgroup
+    assembles det D: every one, interleaved with large batches and with a change
+    of k, equals the large-batch evaluation of the same omegas."""
     from alps_amd.engine import Engine
     p = cases.three_species()
     E = Engine(p)

@@ -88,10 +88,10 @@ def test_series_with_positive_growth_and_far_omegas():
 
 
 def test_series_in_small_batches_and_secant_rounds():
-    """Batches of at most 16 omegas (the request sweep, captured in graphs) and
-    the device-stepped secant rounds sum every row node by node, also after a
-    large batch has built the k's series tables: the same det D and roots with
-    the series switched on and off."""
+    """Batches of at most 16 omegas (the request sweep) and the device-stepped
+    secant rounds sum every row node by node, also after a large batch has built
+    the k's series tables: the same det D and roots with the series switched on
+    and off."""
     from alps_amd.engine import Engine
     p = cases.config1(64, 128)
     om = _map_omegas(16, seed=12)
