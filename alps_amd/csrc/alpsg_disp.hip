@@ -452,11 +452,14 @@ __device__ __forceinline__ void series_row(cdptr c, int J, double zr, double zi,
   for (int k = 0; k < 6; ++k) acc[k] = mk(__builtin_fma(zr, b1[k], __builtin_fma(-sq, b2[k], c[k])), zi * b1[k]);
 }
 
-// The smallest degree J >= 1 at which the series' remainder bound
-// rho^(J+1) / (1 - rho) is below 2^-54 (rho <= SER_RHO < 1).
+// The smallest degree J >= 1 at which the series' remainder, relative to its first
+// term, is at most 2^-53 (rho <= SER_RHO < 1): rho^J / (1 - rho) for the G part, which
+// starts at z, and a factor rho less for the H part.  (A bound on rho^(J+1) left the
+// G part, all that an isotropic species has, short by 2^-54 / rho: electron rows at
+// rho = 7e-5 stopped at z^3, 4e-12 of chi, and det D was up to 5e-11 off.)
 __device__ __forceinline__ int series_degree(double rho) {
-  const double thr = 0x1p-54 * (1.0 - rho);
-  double t = rho * rho;
+  const double thr = 0x1p-53 * (1.0 - rho);
+  double t = rho;
   int J = 1;
   while (t > thr && J < SER_Q - 1) {
     t *= rho;

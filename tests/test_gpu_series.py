@@ -135,3 +135,28 @@ def test_partial_range_rows_in_the_split_form(case, k):
     err = max(abs(one[i] - two[i]) / cases.det_scale(wave[i]) for i in range(om.size))
     print("split vs U/den form:", err, flush=True)
     assert err <= 1e-12
+
+
+@pytest.mark.parametrize("case,kp,kz", [("config1", 0.5, 0.5), ("config1", 0.3, 0.1),
+                                        ("three_species", 0.2, 0.1), ("kappa_case", 0.3, 0.15)])
+def test_series_of_every_degree_to_rounding(case, kp, kz):
+    """|omega| over three decades, so that |m w| / D passes every change of the series'
+    degree: chi of each species with the series and from its nodes.  An isotropic
+    species has no H part, and its G part starts at z, so the remainder counts against
+    that term.  Bar: one rounding per node of either sum."""
+    from alps_amd.engine import Engine
+    p = getattr(cases, case)()
+    E = Engine(p)
+    E.set_k(kp, kz)
+    rng = np.random.default_rng(1)
+    om = np.exp(np.linspace(np.log(2e-3), np.log(2.5), 4096) - 0.3j * rng.uniform(-1, 1, 4096))
+    E.set_shape(om.size, ONE_LANE)
+    on = E.disp_batch(om, want_tensors=True)
+    E.set_sweep_series(False)
+    off = E.disp_batch(om, want_tensors=True)
+    E.close()
+    for j in (1, 2):
+        for s in range(p.nspec):
+            a, b = (np.asarray(x[j])[:, s].reshape(om.size, -1) for x in (on, off))
+            e = np.max(np.abs(a - b), axis=1) / np.max(np.abs(b), axis=1)
+            assert np.max(e) <= p.npar * 2.0 ** -53, (j, s, om[np.argmax(e)], np.max(e))
