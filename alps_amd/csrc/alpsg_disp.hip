@@ -351,9 +351,9 @@ __device__ __forceinline__ void sweep_nodes_pf(cdptr srows, cdptr pa, int npar, 
 
 // The largest cancellation of G/m against C/den that the split form of a row is
 // used at.  256 x 256 omegas of protons and electrons on 128 x 256, shape {1, 2, 4}:
-// at 256, 64, 16, 4 k_sweep takes 454, 483, 478, 588 us, and det D is 5.2e-14, 5.1e-15,
-// 5.1e-15, 5.1e-15 (norm) from the 64-bit sums; the median over points of 15 batches
-// of other sizes and plasmas is 4.4e-15, 3.7e-15, 3.3e-15, 3.1e-15, the last as with
+// at 256, 64, 16, 4 k_sweep takes 472, 481, 485, 588 us, and det D is 5.2e-14, 4.6e-15,
+// 4.6e-15, 4.6e-15 (norm) from the 64-bit sums; the median over points of 15 batches
+// of other sizes and plasmas is 4.2e-15, 3.5e-15, 3.1e-15, 2.9e-15, the last as with
 // the U r products throughout.
 constexpr double SPLIT_MAX = 16.0;
 constexpr int LPA = 1025;  // ppar points a sweep workgroup keeps in LDS (npar <= 1024)

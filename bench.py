@@ -61,18 +61,19 @@ KPERP = KPAR = 0.5
 # batch for every one-lane launch shape (lanes, wavefronts, workgroups per omega
 # block), one counter pass each over `bench.py --pmc-shapes` (far rows summed
 # by their series, after one warm-up batch); a 262144 KiB copy reads
-# FETCH_SIZE 131084-131089 and WRITE_SIZE 262144, so FETCH_SIZE counts half
+# FETCH_SIZE 131084-131094 and WRITE_SIZE 262144, so FETCH_SIZE counts half
 # the bytes fetched and WRITE_SIZE all bytes written.  The writes are the
-# partial-chi slots, 12288 KiB per slot (W x workgroups slots per omega).
+# partial-chi slots, 12288 KiB per slot (W x workgroups slots per omega), and
+# the spilled registers (136 B a lane).
 _SWEEP_PMC_KIB = {
-    (1, 1, 1): (3352.8, 12288.0), (1, 1, 2): (3352.9, 24576.0), (1, 1, 3): (3501.9, 36864.0),
-    (1, 1, 4): (3505.1, 49152.0), (1, 1, 6): (3471.1, 73728.0), (1, 1, 8): (3447.4, 98304.0),
-    (1, 1, 12): (3420.6, 147456.0), (1, 1, 16): (3457.1, 196608.0), (1, 2, 1): (3353.2, 24576.0),
-    (1, 2, 2): (3351.1, 49152.0), (1, 2, 3): (3410.5, 73728.0), (1, 2, 4): (3528.6, 98304.0),
-    (1, 2, 6): (3788.7, 147456.0), (1, 2, 8): (3852.8, 196608.0), (1, 2, 12): (4067.6, 294912.0),
-    (1, 2, 16): (4487.9, 393216.0), (1, 4, 1): (4415.7, 49152.0), (1, 4, 2): (4501.9, 98304.0),
-    (1, 4, 3): (4982.6, 147456.0), (1, 4, 4): (5384.8, 196608.0), (1, 4, 6): (6266.7, 294912.0),
-    (1, 4, 8): (7017.7, 393216.0), (1, 4, 12): (8868.6, 589824.0), (1, 4, 16): (10304.1, 786432.0),
+    (1, 1, 1): (6183.2, 20766.8), (1, 1, 2): (10495.1, 40433.9), (1, 1, 3): (16899.9, 59878.0),
+    (1, 1, 4): (22601.2, 79313.9), (1, 1, 6): (29756.9, 117052.5), (1, 1, 8): (35045.1, 154389.4),
+    (1, 1, 12): (47693.9, 229256.8), (1, 1, 16): (59730.3, 304451.0), (1, 2, 1): (10355.1, 41385.8),
+    (1, 2, 2): (22525.2, 80554.8), (1, 2, 3): (28390.5, 119136.1), (1, 2, 4): (33723.5, 157018.4),
+    (1, 2, 6): (45717.8, 232750.5), (1, 2, 8): (58588.0, 309657.1), (1, 2, 12): (87230.8, 463525.9),
+    (1, 2, 16): (108232.0, 616233.0), (1, 4, 1): (23583.4, 80817.4), (1, 4, 2): (34330.0, 157473.6),
+    (1, 4, 3): (44735.1, 233343.0), (1, 4, 4): (58624.2, 310329.1), (1, 4, 6): (83506.8, 463202.2),
+    (1, 4, 8): (107411.9, 614554.5), (1, 4, 12): (170770.9, 922935.8), (1, 4, 16): (222340.2, 1226715.5),
 }
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0
 SWEEP_TRAFFIC_BYTES = {k: (f * FETCH_SCALE + w * WRITE_SCALE) * 1024.0
@@ -286,8 +287,8 @@ def run_serve_rel(args, seed=5):
     st = S.stats()
     S.close()
     # the relativistic kernels: 55 flops per (point, harmonic) of the 2-D
-    # trapezoid of the non-resonant harmonics (k_rel_nonres) over the time of
-    # both relativistic kernels -- a lower bound: the resonant harmonics'
+    # trapezoid of the non-resonant harmonics (k_rel_nonres_ord) over the time
+    # of all relativistic kernels -- a lower bound: the resonant harmonics'
     # Gamma-row integrals and the resonance scans are not counted
     rel_pts = st["work_rel_points"] - st0["work_rel_points"]
     rel_ms = st["rel_ms"] - st0["rel_ms"]
@@ -327,7 +328,7 @@ def run_serve_rel(args, seed=5):
         "latency_p50_ms": float(np.percentile(lat[conv], 50)) if conv.any() else None,
         "latency_p99_ms": float(np.percentile(lat[conv], 99)) if conv.any() else None,
         "mean_iterations": float(iters.mean()),
-        "roofline_rel": {"kernel": "k_rel_nonres + k_rel_res (all passes)", "bound": "fp64 valu",
+        "roofline_rel": {"kernel": "relativistic kernels (all passes)", "bound": "fp64 valu",
                          "flops_lower_bound": 55.0 * rel_pts, "kernel_ms": rel_ms,
                          "achieved_lower_bound": rel_ach, "peak": FP64_PEAK_TFLOPS,
                          "unit": "TFLOP/s", "frac_lower_bound": rel_ach / FP64_PEAK_TFLOPS,
