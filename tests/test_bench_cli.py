@@ -23,8 +23,9 @@ def test_traffic_table_covers_every_one_lane_shape():
     assert set(bench._SWEEP_PMC_KIB) == shapes
     for (lanes, w, rc), (fetch, write) in bench._SWEEP_PMC_KIB.items():
         # the launch writes one partial chi per omega and slot: 65536 omegas x
-        # 2 species x 6 components x 16 B = 12288 KiB per slot, W RC slots
-        assert write == pytest.approx(12288.0 * w * rc, rel=1e-9)
+        # 2 species x 6 components x 16 B = 12288 KiB per slot, W RC slots; and of
+        # its 136 B of spilled registers per omega and slot (8704 KiB) what leaves L2
+        assert 12288.0 * w * rc <= write <= (12288.0 + 8704.0) * w * rc
         # it reads at least the omegas (1 MiB), i.e. FETCH_SIZE >= 512 KiB at scale 2
         assert fetch * bench.FETCH_SCALE >= 1024.0
         assert bench.SWEEP_TRAFFIC_BYTES[(lanes, w, rc)] == pytest.approx(
