@@ -152,10 +152,11 @@ int alpsg_disp_plain(alpsg_handle h, int n, const double *om, double *det);
 /* alpsg_disp_batch (det only) without any device allocation: no counterpart
    in the reference; for callers that cannot allocate (code under HIP graph
    capture, tight serving loops, harnesses that forbid hipMalloc).  The
-   kernels and launch shape are those of alpsg_disp_batch; the buffers beyond
+   kernels and launch shape are those of alpsg_disp_batch (the shape of the
+   fewest partial sums where an untuned one does not fit); the buffers beyond
    om and det come from a fixed 32 MiB device array per GPU, held until the
-   process ends.  A batch that needs more (n beyond a few thousand omegas,
-   depending on nspec and the launch shape) is refused with ALPSG_E_ARG;
+   process ends.  A batch that needs more (n beyond some 28,000 omegas of two
+   species, fewer in a tuned shape) is refused with ALPSG_E_ARG;
    handles with relativistic or closed-form species with
    ALPSG_E_UNSUPPORTED.  Calls on the handle's device only; calls that
    overlap on one GPU share the array and race, so the caller serialises
